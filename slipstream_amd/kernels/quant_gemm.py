@@ -23,6 +23,9 @@ from slipstream_amd.kernels._common import require_device
 # Split-K partials of the tiled kernel, one buffer per (device, stream): every call writes
 # the partials it reads, so the buffer needs no initialisation and keeps no state.
 _WORKSPACE: dict[tuple[int, int], torch.Tensor] = {}
+# Workspaces that a larger call replaced: a captured graph may still hold their addresses, so
+# they are kept. A new one is at least twice the last, so these are at most as large again.
+_RETIRED: list[torch.Tensor] = []
 # Workspace bytes the library asks for, by shape (a plan depends on the shape and the
 # device's CU count only).
 _WS_NEED: dict[tuple, int] = {}
@@ -34,6 +37,9 @@ def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor |
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     ws = _WORKSPACE.get(key)
     if ws is None or ws.numel() < nbytes:
+        if ws is not None:
+            _RETIRED.append(ws)
+            nbytes = max(nbytes, 2 * ws.numel())
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _WORKSPACE[key] = ws
     return ws

@@ -273,6 +273,41 @@ def test_wide_kernel_two_ranges_graph_and_dirty_workspace(device):
         assert torch.equal(again, y)
 
 
+def test_workspace_growth_keeps_a_captured_graphs_buffer(device):
+    """A call that needs a larger workspace than the stream's must not free the buffer a
+    graph captured earlier writes its partials to: the graph replays to its own result
+    after the growth, a cache trim and a fill of what was freed."""
+    from slipstream_amd.kernels import quant_gemm
+    small = workloads.w4a16_linear(8192, 2048, 64, device=device, seed=1)   # split K, a few MB of partials
+    large = workloads.w4a16_linear(8192, 6144, 256, device=device, seed=2)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+
+    def call(lin):
+        return w4a16_gemm(lin.x, lin.qweight, lin.scales, lin.qzeros, lin.group_size)
+
+    with torch.cuda.stream(st):
+        want = call(small)
+    st.synchronize()
+    key = (torch.device(device).index or 0, st.cuda_stream)
+    before = quant_gemm._WORKSPACE[key]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        out = call(small)
+    with torch.cuda.stream(st):
+        call(large)
+    st.synchronize()
+    after = quant_gemm._WORKSPACE[key]
+    assert after.numel() >= 2 * before.numel() or after is before
+    assert after is before or any(r is before for r in quant_gemm._RETIRED)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 def test_tiled_uneven_ranges_from_the_table_cap(device):
     """K = 15360 at M = 40 over 258 weight tiles: one range per tile would need a 122 KB
     scale table, so the host splits K until a range's table fits 40 KB -- 4 ranges of 32,
