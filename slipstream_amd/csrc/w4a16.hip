@@ -35,166 +35,10 @@
 #include <atomic>
 #include <cstdlib>
 
-#include "ss_common.h"
+#include "w4a16_common.h"
 
 namespace ss {
 namespace {
-
-struct W4Params {
-  const void* x;
-  void* out;
-  const uint32_t* qw;
-  const void* sc;
-  const int32_t* qz;
-  int64_t x_stride, o_stride;  // elements
-  int m, n, k, g, groups, sdt;
-  int kw;  // waves (K slices) per workgroup
-};
-
-constexpr int kMaxKW = 8;
-// Cache policy of the weight loads: non-temporal (every weight is read once per call;
-// streaming without cache allocation measured ~14 % more bandwidth on gfx950).
-constexpr int kNonTemporal = 2;
-// Cache policy sc1 (device scope): a store written through this XCD's L2 to the point of
-// device coherence, a load not served by possibly stale lines of this CU's or XCD's caches.
-constexpr int kDeviceScope = 16;
-
-// s_waitcnt vmcnt(0): every vector memory operation of this wave, stores included, has
-// completed. Inline asm with a memory clobber, so the compiler keeps every load and store
-// written before it on this side of the wait (the waitcnt builtin is not a memory
-// operation, and the stores it must cover could be sunk past it).
-__device__ __forceinline__ void wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// Arrival count of one output tile's K ranges in a 64-bit word: bits 8.. hold the call's
-// tag, bits 0..7 the ranges arrived. A word with another tag (an earlier call, or memory
-// never written) counts as zero arrivals, so the workspace needs no initialisation; the
-// last range resets the word to zero, which the first compare-and-swap of the next call
-// (or of a replayed launch: a captured graph passes the same tag again) expects.
-// No cache maintenance: the partials are device-scope stores the caller has waited for
-// (vmcnt 0) before it arrives, the count is a device-scope atomic, and the last range
-// reads the partials with device-scope loads. (Release/acquire fences at device scope
-// write back or invalidate a whole L2 per wave, several times slower.) This relies on
-// sc1 stores reaching the point of device coherence before their vmcnt decrements, and
-// on sc1 loads not being served by this XCD's possibly stale L2 lines: the gfx950
-// memory model's meaning of the agent-scope cache policy bits.
-__device__ __forceinline__ bool arrive_last(unsigned long long* word, unsigned long long tag, int ranges) {
-  unsigned long long old = 0ull;
-  unsigned long long now;
-  do {
-    const unsigned long long have = (old & ~0xFFull) == tag ? (old & 0xFFull) : 0ull;
-    now = tag | (have + 1);
-  } while (!__hip_atomic_compare_exchange_weak(word, &old, now, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT));
-  if ((int)(now & 0xFFull) != ranges) return false;
-  __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return true;
-}
-
-template <typename T>
-struct W4Elem;
-template <>
-struct W4Elem<bf16_t> {
-  static constexpr uint32_t kMagicPair = 0x43004300u;  // bf16 128.0 in both halves
-  static constexpr uint32_t kOnePair = 0x3F803F80u;    // bf16 1.0 in both halves
-  static constexpr float kMagic = 128.f;
-  static __device__ __forceinline__ float to_f32(uint32_t h) { return __builtin_bit_cast(float, h << 16); }
-};
-template <>
-struct W4Elem<f16_t> {
-  static constexpr uint32_t kMagicPair = 0x64006400u;  // fp16 1024.0 in both halves
-  static constexpr uint32_t kOnePair = 0x3C003C00u;    // fp16 1.0 in both halves
-  static constexpr float kMagic = 1024.f;
-  static __device__ __forceinline__ float to_f32(uint32_t h) {
-    return (float)__builtin_bit_cast(f16_t, (uint16_t)h);
-  }
-};
-
-__device__ __forceinline__ float load_scale(const void* s, int64_t i, int sdt) {
-  if (sdt == SS_DTYPE_F16) return (float)((const f16_t*)s)[i];
-  if (sdt == SS_DTYPE_BF16) return __builtin_bit_cast(float, (uint32_t)((const uint16_t*)s)[i] << 16);
-  return ((const float*)s)[i];
-}
-
-// Scales read without branching on their dtype around the load (a load inside a
-// dtype branch makes the compiler wait for every outstanding load at the join):
-// the aligned dword holding scale gi, through a descriptor bounded by the array
-// (bytes past its end read as zero), shifted so the scale's bits are the low ones;
-// decoded afterwards.
-__device__ __forceinline__ uint32_t scale_bits(__amdgpu_buffer_rsrc_t rs, int64_t gi, int esize) {
-  const int off = (int)(gi * esize);
-  return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, off & ~3, 0, 0) >> (8 * (off & 2));
-}
-__device__ __forceinline__ float decode_scale(uint32_t bits, int sdt) {
-  const float f16 = (float)__builtin_bit_cast(f16_t, (uint16_t)(bits & 0xFFFFu));
-  const float b16 = __builtin_bit_cast(float, bits << 16);
-  return sdt == SS_DTYPE_F16 ? f16 : (sdt == SS_DTYPE_BF16 ? b16 : __builtin_bit_cast(float, bits));
-}
-
-// decode_scale without a branch on the dtype (the branches split the loop body into
-// blocks, and the compiler then sinks whole folds past them, keeping every stage's
-// MFMA partial sums live): all three decodings, merged under uniform bit masks
-// (f16_mask / bf16_mask all-ones for that dtype, else zero).
-__device__ __forceinline__ float decode_scale_masked(uint32_t bits, uint32_t f16_mask, uint32_t bf16_mask) {
-  const uint32_t f16 = __builtin_bit_cast(uint32_t, (float)__builtin_bit_cast(f16_t, (uint16_t)(bits & 0xFFFFu)));
-  const uint32_t b16 = bits << 16;
-  return __builtin_bit_cast(float, (f16 & f16_mask) | (b16 & bf16_mask) | (bits & ~(f16_mask | bf16_mask)));
-}
-
-// Sum over the 16 lanes of a DPP row (every lane of the row gets the total).
-template <int CTRL>
-__device__ __forceinline__ float dpp_f32(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-__device__ __forceinline__ float row16_sum(float x) {
-  x += dpp_f32<0xB1>(x);   // quad_perm [1,0,3,2]
-  x += dpp_f32<0x4E>(x);   // quad_perm [2,3,0,1]
-  x += dpp_f32<0x141>(x);  // row_half_mirror
-  x += dpp_f32<0x140>(x);  // row_mirror
-  return x;
-}
-
-// A constant held in a VGPR. gfx9 VOP3 instructions take no literal and read at most
-// one SGPR, so (w & mask) | magic becomes one v_and_or_b32 only when the magic word
-// already sits in a VGPR (the mask goes to the SGPR slot); otherwise it takes a
-// v_and and a v_or with literals.
-__device__ __forceinline__ uint32_t in_vgpr(uint32_t c) {
-  uint32_t v;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(v) : "s"(c));
-  return v;
-}
-
-// Eight nibbles -> eight 16-bit (MAGIC + q) values in the order k0,k4,k1,k5,k2,k6,k3,k7.
-__device__ __forceinline__ u32x4 nibbles_to_operand(uint32_t w, uint32_t magic) {
-  return u32x4{(w & 0x000F000Fu) | magic, ((w >> 4) & 0x000F000Fu) | magic, ((w >> 8) & 0x000F000Fu) | magic,
-               ((w >> 12) & 0x000F000Fu) | magic};
-}
-
-// Eight consecutive 16-bit x values -> the same order as nibbles_to_operand.
-__device__ __forceinline__ u32x4 permute_x(u32x4 d) {
-  return u32x4{pick_halves<0, 0>(d[0], d[2]), pick_halves<1, 1>(d[0], d[2]), pick_halves<0, 0>(d[1], d[3]),
-               pick_halves<1, 1>(d[1], d[3])};
-}
-
-// acc + a.lo * b.lo + a.hi * b.hi over packed 16-bit pairs, fp32 accumulation
-template <typename T>
-__device__ __forceinline__ float dot2_acc(uint32_t a, uint32_t b, float acc);
-template <>
-__device__ __forceinline__ float dot2_acc<bf16_t>(uint32_t a, uint32_t b, float acc) {
-  typedef short s16x2 __attribute__((ext_vector_type(2)));
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(s16x2, a), __builtin_bit_cast(s16x2, b), acc, false);
-}
-template <>
-__device__ __forceinline__ float dot2_acc<f16_t>(uint32_t a, uint32_t b, float acc) {
-  typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
-  return __builtin_amdgcn_fdot2(__builtin_bit_cast(h16x2, a), __builtin_bit_cast(h16x2, b), acc, false);
-}
-
-// Raw buffer resource over [base, base + bytes): loads past the end return 0, and a
-// per-iteration offset rides in the scalar offset, so the loop does no 64-bit
-// address arithmetic.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
 
 // MT: 16-row activation tiles; NS: 16-row weight tiles; BIT: 128-key iterations
 // per pipeline block; WIDE: g % 128 == 0 (one group per iteration, a lane holds 32
@@ -522,8 +366,6 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
 //     (activation tile, weight tile) pair; one fold per stage:
 //       acc += s * G - s * (MAGIC + z) * X.
 // Every range is a whole number of PF stages (host-checked).
-constexpr int kOutOfRange = 0x40000000;  // buffer offset past any operand (< 2^31 bytes)
-
 template <typename T, int MT, int NS, int PF, int WV>
 __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(2, 2))) void w4a16_tile_kernel(
     const W4Params p, float* __restrict__ part, unsigned long long* __restrict__ arrivals, unsigned long long tag,
@@ -844,77 +686,7 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(2, 2)))
   }
 }
 
-// Eight int4 weights (one word: keys 8j .. 8j + 7 of a row) -> the MFMA B fragment
-// T((q - z) * s) in key order, computed as fma(q, s, -z s) in fp32 and rounded once
-// to the activation type. (The reference rounds (q - z) * s to the scales' dtype and
-// then to the activation dtype, quant_ref.py:112-116,132; with fp16 scales and bf16
-// activations the single rounding differs from that double rounding by at most one
-// bf16 ulp of a weight.) Per word: two masks, eight byte converts (v_cvt_f32_ubyteN),
-// eight FMAs and four packs.
-template <typename T>
-__device__ __forceinline__ u32x4 dequant_word(uint32_t w, float s, float nzs) {
-  // the masks as asm, so that the compiler does not fold each (lo >> 8b) & 0xFF into a
-  // 4-bit field extract and lose the byte converts' own byte select
-  uint32_t lo, hi;
-  asm("v_and_b32 %0, 0x0f0f0f0f, %1" : "=v"(lo) : "v"(w));
-  asm("v_and_b32 %0, 0x0f0f0f0f, %1" : "=v"(hi) : "v"(w >> 4));
-  u32x4 r;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const float qa = (float)((lo >> (8 * b)) & 0xFFu), qb = (float)((hi >> (8 * b)) & 0xFFu);
-    r[b] = Elem<T>::pack2(fmaf(qa, s, nzs), fmaf(qb, s, nzs));
-  }
-  return r;
-}
-
-// Scale of SD (a dtype code) from its raw bits (the low 16 bits for 16-bit scales).
-template <int SD>
-__device__ __forceinline__ float scale_from_bits(uint32_t b) {
-  if constexpr (SD == SS_DTYPE_F16) return (float)__builtin_bit_cast(f16_t, (uint16_t)(b & 0xFFFFu));
-  if constexpr (SD == SS_DTYPE_BF16) return __builtin_bit_cast(float, b << 16);
-  return __builtin_bit_cast(float, b);
-}
-
 constexpr int kWideMT = 8, kWideNS = 2, kWideWV = 8, kWidePF = 4;
-
-// Buffer loads for the wide kernel, written as asm: the compiler inserts no vmcnt wait
-// of its own for them (its count of loads in flight, merged around the loop's back
-// edge, made it wait for nearly every prefetched stage at the top of each stage). The
-// kernel waits itself, with vm_wait_tied, whose register operands keep every use of a
-// loaded value behind the wait. Descriptors are plain SGPR quads over [base, base + bytes):
-// offsets past the end read zeros without a memory access.
-typedef int i32x4w __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ i32x4w wide_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t a = (uint64_t)base;
-  return i32x4w{(int)(uint32_t)a, (int)((uint32_t)(a >> 32) & 0xFFFF), (int)bytes, 0x00020000};
-}
-__device__ __forceinline__ u32x4 asm_load_b128_nt(i32x4w rs, int voff, int soff) {
-  u32x4 v;
-  asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen nt" : "=v"(v) : "v"(voff), "s"(rs), "s"(soff));
-  return v;
-}
-__device__ __forceinline__ uint32_t asm_load_b32(i32x4w rs, int voff) {
-  uint32_t v;
-  asm volatile("buffer_load_dword %0, %1, %2, 0 offen" : "=v"(v) : "v"(voff), "s"(rs));
-  return v;
-}
-__device__ __forceinline__ uint32_t asm_load_u16(i32x4w rs, int voff) {
-  uint32_t v;
-  asm volatile("buffer_load_ushort %0, %1, %2, 0 offen" : "=v"(v) : "v"(voff), "s"(rs));
-  return v;
-}
-
-// 16 bytes per lane from rs + voff + soff straight into LDS at lds + 16 * lane
-// (buffer_load_dwordx4 ... lds; M0 holds the LDS destination). The s_nop: M0 is
-// written just before by the compiler, and the load may read it one wait state later.
-typedef __attribute__((address_space(3))) char* LdsW;
-__device__ __forceinline__ void asm_dma_b128(i32x4w rs, LdsW lds, int voff, int soff) {
-  const uint32_t m0 = (uint32_t)(uintptr_t)lds;
-  asm volatile("s_nop 1\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-               :
-               : "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0)
-               : "memory");
-}
 
 // s_waitcnt vmcnt(N) with the registers of one stage's weight loads as operands, so
 // that no use of them is scheduled above the wait.
@@ -1831,6 +1603,8 @@ struct W4Plan {
   bool skinny;  // the skinny kernel (m <= 64, K split over the waves of one workgroup)
   bool widek;   // the wide kernel (m > 64, weights dequantised once per wave)
   int st;       // skinny: 128-key stages per wave
+  bool panel;   // the panel kernel (m > 64, the matrix cores' shapes)
+  PanelPlan pp;
   int mt, ns, bit, kw, pf;
   int m_blocks, n_tiles;
   int ks, kchunk;  // tiled kernel: K ranges and 128-key stages per range
@@ -1986,6 +1760,7 @@ bool plan_skinny(W4Plan& pl, int64_t m, int64_t n, int64_t k, int g) {
 // The wide kernel's: the partials alone.
 int64_t tile_part_bytes(const W4Plan& pl, int64_t m, int64_t n) { return ((int64_t)pl.ks * m * n * 4 + 255) / 256 * 256; }
 int64_t tile_workspace_bytes(const W4Plan& pl, int64_t m, int64_t n) {
+  if (pl.panel) return pl.ks > 1 ? tile_part_bytes(pl, m, n) : 0;
   if (pl.widek) return pl.ks > 1 ? tile_part_bytes(pl, m, n) + (int64_t)pl.n_tiles * pl.m_blocks * 8 : 0;
   return pl.tile && pl.ks > 1 ? tile_part_bytes(pl, m, n) + (int64_t)pl.n_tiles * pl.m_blocks * 8 : 0;
 }
@@ -2046,7 +1821,7 @@ bool plan_wide(W4Plan& pl, int64_t m, int64_t n, int64_t k, int g) {
 
 constexpr size_t kLdsBudget = 64 * 1024;  // LDS bytes per workgroup
 
-W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow_tile = true) {
+W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow_tile = true, bool allow_panel = true) {
   W4Plan pl = {};
   pl.fast = act16 && k % 128 == 0 && g % 32 == 0 && k > 0 && n * k / 2 < ((int64_t)1 << 31);
   pl.wide = g % 128 == 0;
@@ -2076,7 +1851,21 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
     }
   }
   if (plan_skinny(pl, m, n, k, g)) return pl;
-  if (allow_tile && plan_wide(pl, m, n, k, g)) return pl;
+  if (allow_tile && plan_wide(pl, m, n, k, g)) {
+    // the panel kernel (weights rounded to the operand type in the same way) where its
+    // taller tiles come out ahead. The wide kernel takes 2.15 us a stage and round of one
+    // workgroup per CU (m = 197 and 512 x 4096 x 28672: 2.2 us).
+    const int64_t cus = ss_host::device_cu_count();
+    const int64_t rounds = ((int64_t)pl.ks * pl.n_tiles * pl.m_blocks + cus - 1) / cus;
+    double t = (double)rounds * (2.15 * pl.kchunk * pl.ns / kWideNS + 4.0);
+    if (pl.ks > 1) t += (double)pl.ks * (double)m * (double)n * 8e-6 / 4.0 + 4.0;
+    if (allow_panel && plan_w4a16_panel(pl.pp, m, n, k, g, t)) {
+      pl.widek = false;
+      pl.panel = true;
+      pl.ks = pl.pp.ks, pl.m_blocks = pl.pp.m_blocks, pl.n_tiles = pl.pp.n_tiles;
+    }
+    return pl;
+  }
   pl.widek = false;
   if (allow_tile && plan_tile(pl, m, n, k, g)) return pl;
   pl.tile = false;
@@ -2140,6 +1929,21 @@ unsigned long long next_arrival_tag() {
 
 // NS weight tiles per wave, WV waves: the plan's 64 * pl.ns rows per workgroup are
 // 16 * NS * WV
+// The K ranges' partials added in range order into the output.
+template <typename T>
+int launch_splitk_reduce(const W4Params& p, int ks, const float* part, hipStream_t stream) {
+  const bool vec = p.n % 4 == 0;
+  const int64_t threads = (int64_t)p.m * (vec ? p.n / 4 : p.n);
+  const unsigned blocks = (unsigned)((threads + 255) / 256);
+  if (vec)
+    hipLaunchKernelGGL((w4a16_splitk_reduce_kernel<T, 4>), dim3(blocks), dim3(256), 0, stream, part, p.out, p.m, p.n,
+                       ks, p.o_stride);
+  else
+    hipLaunchKernelGGL((w4a16_splitk_reduce_kernel<T, 1>), dim3(blocks), dim3(256), 0, stream, part, p.out, p.m, p.n,
+                       ks, p.o_stride);
+  return ss_host::launch_status("w4a16 split-K reduce");
+}
+
 template <typename T, int MT, int NS, int PF, int WV>
 int launch_w4a16_tile(const W4Params& p, const W4Plan& pl, float* part, hipStream_t stream) {
   if (16 * NS * WV != 64 * pl.ns) {
@@ -2177,16 +1981,7 @@ int launch_w4a16_tile(const W4Params& p, const W4Plan& pl, float* part, hipStrea
                      part, arrivals, tag, pl.kchunk, pl.ks, pl.n_tiles, pl.m_blocks);
   int st = ss_host::launch_status("w4a16 gemm (tiled)");
   if (st != SS_OK || pl.ks == 1 || fused) return st;
-  const bool vec = p.n % 4 == 0;
-  const int64_t threads = (int64_t)p.m * (vec ? p.n / 4 : p.n);
-  const unsigned blocks = (unsigned)((threads + 255) / 256);
-  if (vec)
-    hipLaunchKernelGGL((w4a16_splitk_reduce_kernel<T, 4>), dim3(blocks), dim3(256), 0, stream, part, p.out, p.m, p.n,
-                       pl.ks, p.o_stride);
-  else
-    hipLaunchKernelGGL((w4a16_splitk_reduce_kernel<T, 1>), dim3(blocks), dim3(256), 0, stream, part, p.out, p.m, p.n,
-                       pl.ks, p.o_stride);
-  return ss_host::launch_status("w4a16 split-K reduce");
+  return launch_splitk_reduce<T>(p, pl.ks, part, stream);
 }
 
 template <typename T, int MT, int NS, int ST>
@@ -2306,16 +2101,7 @@ int launch_w4a16_wide_sd(const W4Params& p, const W4Plan& pl, float* part, hipSt
                      pl.ks, pl.n_tiles, pl.m_blocks);
   int st = ss_host::launch_status("w4a16 gemm (wide)");
   if (st != SS_OK || pl.ks == 1 || fused) return st;
-  const bool vec = p.n % 4 == 0;
-  const int64_t threads = (int64_t)p.m * (vec ? p.n / 4 : p.n);
-  const unsigned blocks = (unsigned)((threads + 255) / 256);
-  if (vec)
-    hipLaunchKernelGGL((w4a16_splitk_reduce_kernel<T, 4>), dim3(blocks), dim3(256), 0, stream, part, p.out, p.m, p.n,
-                       pl.ks, p.o_stride);
-  else
-    hipLaunchKernelGGL((w4a16_splitk_reduce_kernel<T, 1>), dim3(blocks), dim3(256), 0, stream, part, p.out, p.m, p.n,
-                       pl.ks, p.o_stride);
-  return ss_host::launch_status("w4a16 split-K reduce");
+  return launch_splitk_reduce<T>(p, pl.ks, part, stream);
 }
 
 template <typename T>
@@ -2410,6 +2196,10 @@ extern "C" int ss_w4a16_workspace_size(int64_t m, int64_t n, int64_t k, int grou
   }
   const ss::W4Plan pl = ss::plan_w4a16(m, n, k, group_size, act_dtype != SS_DTYPE_F32);
   *bytes = pl.fast ? ss::tile_workspace_bytes(pl, m, n) : 0;
+  if (pl.panel) {  // fp32 scales or rows too far apart take the wide kernel's plan
+    const int64_t other = ss::tile_workspace_bytes(ss::plan_w4a16(m, n, k, group_size, true, true, false), m, n);
+    if (other > *bytes) *bytes = other;
+  }
   return SS_OK;
 }
 
@@ -2445,21 +2235,26 @@ extern "C" int ss_w4a16_gemm(const void* x, void* out, const int32_t* qweight, c
   p.groups = (int)(k / group_size);
   p.sdt = scale_dtype;
   const bool act16 = act_dtype != SS_DTYPE_F32;
-  ss::W4Plan pl = ss::plan_w4a16(m, n, k, group_size, act16);
+  // the panel kernel: 16-bit scales (its fp16 bias trick is exact for those), 32-bit byte
+  // offsets over 256 activation rows
+  const bool panel = scale_dtype != SS_DTYPE_F32 && ((int64_t)255 * x_stride + k) * 2 < ((int64_t)1 << 31);
+  ss::W4Plan pl = ss::plan_w4a16(m, n, k, group_size, act16, true, panel);
   if (pl.fast && (!aligned16(x) || x_stride % 8 != 0 || !aligned16(qweight))) pl.fast = false;
   // activation fragments are addressed by 32-bit byte offsets within a 64-row block
   if (pl.fast && ((int64_t)63 * x_stride + k) * 2 >= ((int64_t)1 << 31)) pl.fast = false;
   // scale and zero-point offsets are 32-bit byte offsets
   if (pl.fast && n * (k / group_size) * 4 >= ((int64_t)1 << 31)) pl.fast = false;
-  if (pl.fast && (pl.tile || pl.widek) && pl.ks > 1) {
-    // the K split needs the workspace ss_w4a16_workspace_size reports; without it
-    // (or unaligned) the untiled MFMA kernel runs, which needs none
-    const int64_t need = ss::tile_workspace_bytes(pl, m, n);
-    if (!workspace || workspace_bytes < need || !aligned16(workspace)) {
-      const bool fast = pl.fast;
-      pl = ss::plan_w4a16(m, n, k, group_size, act16, false);
-      pl.fast = pl.fast && fast;
-    }
+  if (pl.fast && (pl.tile || pl.widek || pl.panel) && pl.ks > 1) {
+    // the K split needs the workspace ss_w4a16_workspace_size reports; without it (or
+    // unaligned) the wide kernel's plan if it does not split, else the untiled MFMA
+    // kernel, which need none
+    const bool fast = pl.fast;
+    auto short_of = [&](const ss::W4Plan& q) {
+      return q.ks > 1 && (!workspace || workspace_bytes < ss::tile_workspace_bytes(q, m, n) || !aligned16(workspace));
+    };
+    if (short_of(pl) && pl.panel) pl = ss::plan_w4a16(m, n, k, group_size, act16, true, false);
+    if (short_of(pl)) pl = ss::plan_w4a16(m, n, k, group_size, act16, false);
+    pl.fast = pl.fast && fast;
   }
   hipStream_t s = (hipStream_t)stream;
   if (!pl.fast) {
@@ -2483,6 +2278,12 @@ extern "C" int ss_w4a16_gemm(const void* x, void* out, const int32_t* qweight, c
   }
   p.kw = pl.kw;
   float* part = (float*)workspace;
+  if (pl.panel) {
+    st = ss::launch_w4a16_panel(p, pl.pp, act_dtype, part, s);
+    if (st != SS_OK || pl.ks == 1) return st;
+    return act_dtype == SS_DTYPE_BF16 ? ss::launch_splitk_reduce<ss::bf16_t>(p, pl.ks, part, s)
+                                      : ss::launch_splitk_reduce<ss::f16_t>(p, pl.ks, part, s);
+  }
   if (act_dtype == SS_DTYPE_BF16) return ss::launch_w4a16_typed<ss::bf16_t>(p, pl, part, s);
   return ss::launch_w4a16_typed<ss::f16_t>(p, pl, part, s);
 }

@@ -238,6 +238,40 @@ def test_wide_kernel(device, m, k, n, act, sdt):
     assert torch.equal(w4a16_gemm(xs, qd, sd, zd, 128), y)  # strided activations: the same result
 
 
+# (plans as the host computes them for 256 CUs: panels of 16 MT rows, 256-row weight tiles)
+@pytest.mark.parametrize("m,k,n,act,sdt", [
+    (150, 2048, 20480, torch.float16, torch.bfloat16),   # MT 8, the last panel of 22 rows
+    (420, 2048, 20480, torch.bfloat16, torch.float16),   # MT 10, the last panel of 100 rows
+    (520, 2048, 20480, torch.bfloat16, torch.bfloat16),  # MT 12
+    (600, 2048, 20490, torch.float16, torch.float16),    # MT 14, the last weight tile of 10 rows
+    (500, 2048, 28600, torch.bfloat16, torch.float16),   # MT 16, N % 256 = 184
+    (150, 8192, 4100, torch.bfloat16, torch.float16),    # eight K ranges of 8 stages, a weight tile of 4 rows
+    (180, 4096, 8200, torch.bfloat16, torch.float16),    # three K ranges of 11, 11 and 10 stages
+    (600, 4096, 8190, torch.bfloat16, torch.float16),    # two K ranges, N % 4 != 0: element stores of the partials
+    (513, 2048, 16002, torch.bfloat16, torch.float16),   # N % 8 != 0: element stores of the results, one row in the last panel
+    (420, 2048, 20480, torch.bfloat16, torch.float32),   # fp32 scales: the wide kernel
+])
+def test_panel_kernel(device, m, k, n, act, sdt):
+    """The panel kernel (panels of 128 to 256 activation rows, weights dequantised once per
+    workgroup): every panel height, ragged M and N, K ranges of unequal length, both
+    activation and 16-bit scale dtypes, random zero points, strided activations and
+    outputs of a workspace full of 0xFF. Within the tolerance of the float64 oracle,
+    bit-identical across repeats."""
+    from slipstream_amd.kernels import quant_gemm
+    print(f"w4a16 panel m={m} k={k} n={n} {act} {sdt}", flush=True)
+    x, qw, s, z, ref = _host_case(n, k, m, 128, seed=m + k + n, act=act, sdt=sdt, zeros="random")
+    xd, qd, sd, zd = x.to(device), qw.to(device), s.to(device), z.to(device)
+    y = w4a16_gemm(xd, qd, sd, zd, 128)
+    assert y.dtype == act
+    _assert_close(y, ref, f"panel m={m} k={k} n={n}")
+    for ws in quant_gemm._WORKSPACE.values():
+        ws.fill_(0xFF)
+    assert torch.equal(y, w4a16_gemm(xd, qd, sd, zd, 128))
+    xs = torch.zeros(m, k + 72, dtype=act, device=device)[:, 40:40 + k]  # rows 16-byte aligned, stride k + 72
+    xs.copy_(xd)
+    assert torch.equal(w4a16_gemm(xs, qd, sd, zd, 128), y)
+
+
 def test_wide_kernel_two_ranges_graph_and_dirty_workspace(device):
     """The wide kernel's in-kernel finish of two K ranges (arrival words behind the
     partials, tagged per call): correct on a workspace full of 0xFF bytes and replayed
