@@ -16,7 +16,7 @@
 // (k0,k4),(k1,k5),(k2,k6),(k3,k7) of each word, and every activation fragment is
 // permuted the same way in registers (v_perm_b32), so the dot products pair up.
 //
-// Untiled kernel (w4a16_kernel): a workgroup owns 16*NS weight rows and 16*MT
+// Untiled kernel (w4a16_kernel, m > 32 where the tiled kernels do not take the shape): a workgroup owns 16*NS weight rows and 16*MT
 // activation rows; its KW waves split K into contiguous slices (each wave streams
 // its own slice of the rows: coalesced 16-byte loads, the next block in flight
 // while the current one computes), and one LDS pass adds the slices in wave
@@ -29,6 +29,10 @@
 // through LDS; K is split over workgroups and a second kernel adds the fp32
 // partials in range order. Batch 1 takes a bandwidth GEMV. In every case the
 // result does not depend on timing.
+//
+// Group kernel (w4a16_group.hip): m <= 32 with groups of 32 or 64 keys, or a number of
+// stages the skinny and tiled kernels do not split. Panel kernel (w4a16_panel.hip): m > 64
+// where the matrix cores set the time.
 //
 // Generic path (any other shape, fp32 activations): one thread per output,
 // fp32 dequant and dot product.
@@ -43,18 +47,14 @@ namespace {
 // MT: 16-row activation tiles; NS: 16-row weight tiles; BIT: 128-key iterations
 // per pipeline block; WIDE: g % 128 == 0 (one group per iteration, a lane holds 32
 // consecutive keys of its row: one 16-byte load), else g % 32 == 0 (one group per
-// 32-key MFMA step, 4-byte loads); XLDS: the workgroup's activation rows (all of K,
-// permuted) and their per-fold sums are staged in LDS once -- used when they fit;
-// otherwise every wave loads its own activation fragments and sums them with an
-// all-ones MFMA.
+// 32-key MFMA step, 4-byte loads). Every wave loads its own activation fragments and sums
+// them with an all-ones MFMA.
 //
-// Dynamic LDS: [XLDS: x rows (K + 8 elements each) | fold sums [K/UNIT][16*MT]]
-//              [scale table: 16*NS rows x (2*groups + 2) floats, pairs (s, s*(MAGIC+z))]
+// Dynamic LDS: the scale table, 16*NS rows x (2*groups + 2) floats, pairs (s, s*(MAGIC+z)),
 // and, once every wave is past the main loop, the same bytes again as the
 // reduction buffer (kw - 1) x MT*NS x 64 x f32x4.
-template <typename T, int MT, int NS, int BIT, bool WIDE, bool XLDS>
+template <typename T, int MT, int NS, int BIT, bool WIDE>
 __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
-  constexpr int UNIT = WIDE ? 128 : 32;  // keys per fold (one quantisation group; 4 per 128-key iteration if !WIDE)
   typedef W4Elem<T> E;
   extern __shared__ __attribute__((aligned(16))) char s_dyn[];
 
@@ -70,14 +70,10 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
   const int per = (iters + p.kw - 1) / p.kw;
   const int it0 = wave * per;
   const int it1 = min(iters, it0 + per);
-  const int lrow = p.k + 8;           // LDS row of x, elements (16-byte skew per row)
   const int szrow = 2 * p.groups + 2;  // LDS row of the scale table, floats (8-byte skew per row)
   const uint32_t magic = in_vgpr(E::kMagicPair);
 
-  T* s_x = (T*)s_dyn;
-  const size_t x_bytes = XLDS ? (size_t)rows * lrow * sizeof(T) + (size_t)(p.k / UNIT) * 16 * MT * 4 : 0;
-  float* s_xs = (float*)(s_dyn + (XLDS ? (size_t)rows * lrow * sizeof(T) : 0));
-  float* s_sz = (float*)(s_dyn + x_bytes);
+  float* s_sz = (float*)s_dyn;
   f32x4* s_red = (f32x4*)s_dyn;  // aliases the tables above, used after a barrier
 
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(p.qw, (uint32_t)((int64_t)p.n * p.k / 2));
@@ -92,7 +88,7 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
     u32x4 w[NS][BIT];
   };
   struct XBlock {
-    u32x4 x[XLDS ? 1 : MT][XLDS ? 1 : BIT][4];
+    u32x4 x[MT][BIT][4];
   };
 
   // Weight loads only (no use), always in range: iterations past the slice reload
@@ -150,25 +146,6 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
       }
     }
   }
-  if (XLDS) {
-    // rows [m0, m0 + rows) of x for all of K, permuted, plus their fold sums
-    constexpr int GL = UNIT / 8;  // staging lanes per fold (consecutive lanes)
-    const int cols = p.k / 8;
-    for (int q = threadIdx.x; q < rows * cols; q += blockDim.x) {
-      const int r = q / cols, c = q - r * cols;
-      const u32x4 v = load16((const T*)p.x + (int64_t)(m0 + r) * p.x_stride + 8 * c);
-      store16(&s_x[r * lrow + 8 * c], permute_x(v));
-      float sum = 0.f;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sum += E::to_f32(v[j] & 0xFFFFu) + E::to_f32(v[j] >> 16);
-#pragma unroll
-      for (int o = 1; o < GL; o <<= 1) sum += __shfl_xor(sum, o);
-      if (c % GL == 0) s_xs[(c / GL) * 16 * MT + r] = sum;
-    }
-    // sums of rows past M are 0 (their outputs are never stored)
-    for (int q = threadIdx.x; q < (p.k / UNIT) * 16 * MT; q += blockDim.x)
-      if (q % (16 * MT) >= rows) s_xs[q] = 0.f;
-  }
   __syncthreads();
 
   // Activation rows past M read row M-1 (a valid address); they only feed output
@@ -181,11 +158,9 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
   const __amdgpu_buffer_rsrc_t rx = buffer_rsrc(
       (const T*)p.x + (int64_t)m0 * p.x_stride, (uint32_t)(((int64_t)(rows - 1) * p.x_stride + p.k) * sizeof(T)));
   int xrow[MT];  // byte offset of this lane's activation row
-  int xl[MT];    // LDS row (XLDS)
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     xrow[mt] = (int)((int64_t)min(mt * 16 + ln, rows - 1) * p.x_stride * (int64_t)sizeof(T));
-    xl[mt] = min(mt * 16 + ln, rows - 1) * lrow;
   }
 
   f32x4 acc[MT][NS];
@@ -195,7 +170,6 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
     for (int ns = 0; ns < NS; ++ns) acc[mt][ns] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   auto load_x = [&](int itb, XBlock& xb) {
-    if (XLDS) return;
 #pragma unroll
     for (int it = 0; it < BIT; ++it) {
       // the iteration's key offset is uniform: it rides in the scalar offset, so the
@@ -207,7 +181,7 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
         const int klane = (WIDE ? 32 * kg + 8 * s : 32 * s + 8 * kg) * (int)sizeof(T);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
-          xb.x[XLDS ? 0 : mt][XLDS ? 0 : it][s] = __builtin_bit_cast(
+          xb.x[mt][it][s] = __builtin_bit_cast(
               u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xrow[mt] + klane, kk, 0));
       }
     }
@@ -233,12 +207,8 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
         u32x4 a[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          if (XLDS) {
-            a[mt] = load16(&s_x[xl[mt] + kk + (WIDE ? 32 * kg + 8 * s : 32 * s + 8 * kg)]);
-          } else {
-            a[mt] = permute_x(xb.x[XLDS ? 0 : mt][XLDS ? 0 : it][s]);
-            X[mt] = Elem<T>::mfma(a[mt], ones, X[mt]);
-          }
+          a[mt] = permute_x(xb.x[mt][it][s]);
+          X[mt] = Elem<T>::mfma(a[mt], ones, X[mt]);
         }
 #pragma unroll
         for (int ns = 0; ns < NS; ++ns) {
@@ -248,11 +218,6 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
         }
         if (!WIDE || s == 3) {  // end of a fold unit: fold it into acc
           const int kf = kk + (WIDE ? 0 : 32 * s);
-          if (XLDS) {
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              X[mt] = *reinterpret_cast<const f32x4*>(&s_xs[(kf / UNIT) * 16 * MT + mt * 16 + 4 * kg]);
-          }
           const int gi = kf / p.g;
 #pragma unroll
           for (int ns = 0; ns < NS; ++ns) {
@@ -1596,7 +1561,6 @@ __global__ __launch_bounds__(512) void w4a16_narrow_kernel(const W4Params p) {
 struct W4Plan {
   bool fast;
   bool wide;
-  bool xlds;
   int narrow;  // activation rows of the narrow kernel (1, 2 or 4), 0: not used
   int gemv;  // 1: the batch-1 GEMV kernel
   bool tile;  // the tiled kernel (activations shared through LDS)
@@ -1605,7 +1569,9 @@ struct W4Plan {
   int st;       // skinny: 128-key stages per wave
   bool panel;   // the panel kernel (m > 64, the matrix cores' shapes)
   PanelPlan pp;
-  int mt, ns, bit, kw, pf;
+  bool group;   // the group kernel (m <= 64, groups of 32 or 64, or stages the others cannot split)
+  GroupPlan gp;
+  int mt, ns, kw, pf;
   int m_blocks, n_tiles;
   int ks, kchunk;  // tiled kernel: K ranges and 128-key stages per range
   size_t lds;
@@ -1869,30 +1835,10 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
   pl.widek = false;
   if (allow_tile && plan_tile(pl, m, n, k, g)) return pl;
   pl.tile = false;
-  const size_t unit = pl.wide ? 128 : 32;
   const int64_t groups = k / g;
   const int iters = (int)(k / 128);
   const int64_t want = 8LL * ss_host::device_cu_count();  // waves in flight to cover HBM latency
-  // x staged in LDS when one 16-row tile of it fits beside the scale table
-  const int64_t rows1 = m < 16 ? m : 16;
-  const size_t x1 = (size_t)rows1 * (k + 8) * 2 + (size_t)(k / unit) * 16 * 4;
-  const size_t sz1 = (size_t)16 * (2 * groups + 2) * 4;
-  if (m <= 16 && x1 + sz1 <= kLdsBudget) {
-    pl.mt = 1, pl.ns = 1, pl.bit = 4, pl.xlds = true;
-  } else if (m <= 16) {
-    // 64 weight rows share each activation fragment, unless that leaves more than
-    // half the CUs idle: then 32 (twice the activation reads, twice the workgroups;
-    // measured faster for N = 4096 and 6144, slower for 14336)
-    const int64_t cus = ss_host::device_cu_count();
-    if ((n + 63) / 64 >= cus / 2)
-      pl.mt = 1, pl.ns = 4, pl.bit = 2;
-    else
-      pl.mt = 1, pl.ns = 2, pl.bit = 2;
-  } else if (m <= 32) {
-    pl.mt = 2, pl.ns = 2, pl.bit = 2;
-  } else {
-    pl.mt = 4, pl.ns = 2, pl.bit = 1;
-  }
+  pl.mt = 4, pl.ns = 2;
   pl.m_blocks = (int)((m + 16 * pl.mt - 1) / (16 * pl.mt));
   pl.n_tiles = (int)((n + 16 * pl.ns - 1) / (16 * pl.ns));
   // K slices per workgroup, with at least two 128-key iterations per slice
@@ -1900,21 +1846,28 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
   pl.kw = wgs * 4 >= want ? 4 : kMaxKW;
   while (pl.kw > 1 && iters < 2 * pl.kw) pl.kw >>= 1;
   const size_t red = (size_t)(pl.kw - 1) * pl.mt * pl.ns * 64 * 16;
-  const size_t xb = pl.xlds ? x1 : 0;
   const size_t szb = (size_t)16 * pl.ns * (2 * groups + 2) * 4;
-  pl.lds = xb + szb > red ? xb + szb : red;  // the reduction reuses the tables' bytes
-  if (pl.lds > kLdsBudget) pl.fast = false;  // scale table too large: scalar kernel
+  pl.lds = szb > red ? szb : red;  // the reduction reuses the table's bytes
+  // the group kernel up to 32 rows, above them for N <= 4096 (m = 64, g = 64: 4864 x 896
+  // 24.6 against 35.5 us, 14336 x 4096 70 against 93; m = 40, 4096 x 6144 32 against 28),
+  // and where the scale table does not fit (m = 16, g = 32, 14336 x 4096 on the scalar
+  // kernel 1460 us, here 27)
+  if ((m <= 32 || n <= 4096 || pl.lds > kLdsBudget) && plan_w4a16_group(pl.gp, m, n, k, g)) {
+    pl.group = true;
+    pl.m_blocks = pl.gp.m_blocks;
+  }
+  if (pl.lds > kLdsBudget && (!pl.group || pl.m_blocks > 65535)) pl.fast = false;  // scalar kernel
   return pl;
 }
 
-template <typename T, int MT, int NS, int BIT, bool X>
-int launch_w4a16_x(const W4Params& p, const W4Plan& pl, hipStream_t stream) {
+template <typename T>
+int launch_w4a16_untiled(const W4Params& p, const W4Plan& pl, hipStream_t stream) {
   dim3 grid((unsigned)pl.n_tiles, (unsigned)pl.m_blocks);
   dim3 block(64 * pl.kw);
   if (pl.wide)
-    hipLaunchKernelGGL((w4a16_kernel<T, MT, NS, BIT, true, X>), grid, block, pl.lds, stream, p);
+    hipLaunchKernelGGL((w4a16_kernel<T, 4, 2, 1, true>), grid, block, pl.lds, stream, p);
   else
-    hipLaunchKernelGGL((w4a16_kernel<T, MT, NS, BIT, false, X>), grid, block, pl.lds, stream, p);
+    hipLaunchKernelGGL((w4a16_kernel<T, 4, 2, 1, false>), grid, block, pl.lds, stream, p);
   return ss_host::launch_status("w4a16 gemm");
 }
 
@@ -2144,11 +2097,7 @@ int launch_w4a16_typed(const W4Params& p, const W4Plan& pl, float* part, hipStre
                          dim3((unsigned)(64 * (p.k / 2048))), pl.lds, stream, p);
     return ss_host::launch_status("w4a16 gemv");
   }
-  if (pl.xlds) return launch_w4a16_x<T, 1, 1, 4, true>(p, pl, stream);
-  if (pl.mt == 1 && pl.ns == 4) return launch_w4a16_x<T, 1, 4, 2, false>(p, pl, stream);
-  if (pl.mt == 1) return launch_w4a16_x<T, 1, 2, 2, false>(p, pl, stream);
-  if (pl.mt == 2) return launch_w4a16_x<T, 2, 2, 2, false>(p, pl, stream);
-  return launch_w4a16_x<T, 4, 2, 1, false>(p, pl, stream);
+  return launch_w4a16_untiled<T>(p, pl, stream);
 }
 
 }  // namespace
@@ -2278,6 +2227,7 @@ extern "C" int ss_w4a16_gemm(const void* x, void* out, const int32_t* qweight, c
   }
   p.kw = pl.kw;
   float* part = (float*)workspace;
+  if (pl.group) return ss::launch_w4a16_group(p, pl.gp, act_dtype, s);
   if (pl.panel) {
     st = ss::launch_w4a16_panel(p, pl.pp, act_dtype, part, s);
     if (st != SS_OK || pl.ks == 1) return st;

@@ -23,6 +23,14 @@ struct PanelPlan {
   int ks, kchunk;  // K ranges and 128-key stages per range
   int n_tiles, m_blocks;
 };
+// The group kernel (w4a16_group.hip): tiles, waves and stages per wave of a workgroup.
+struct GroupPlan {
+  int mt, ns, waves, per;
+  int n_tiles, m_blocks;
+};
+bool plan_w4a16_group(GroupPlan& pl, int64_t m, int64_t n, int64_t k, int g);
+int launch_w4a16_group(const W4Params& p, const GroupPlan& pl, int act_dtype, hipStream_t stream);
+
 bool plan_w4a16_panel(PanelPlan& pl, int64_t m, int64_t n, int64_t k, int g, double other);
 int launch_w4a16_panel(const W4Params& p, const PanelPlan& pl, int act_dtype, float* part, hipStream_t stream);
 

@@ -238,6 +238,36 @@ def test_wide_kernel(device, m, k, n, act, sdt):
     assert torch.equal(w4a16_gemm(xs, qd, sd, zd, 128), y)  # strided activations: the same result
 
 
+@pytest.mark.parametrize("m,k,n,g,act,sdt", [
+    (1, 128, 16, 32, torch.bfloat16, torch.float16),       # one stage, one wave, one row
+    (11, 896, 9728, 64, torch.float16, torch.float16),     # two weight tiles, four waves, a run of one stage
+    (16, 4864, 900, 64, torch.bfloat16, torch.bfloat16),   # thirteen waves of three stages, N % 16 = 4
+    (3, 2432, 24600, 64, torch.bfloat16, torch.float32),   # four weight tiles, the last of 24 rows
+    (16, 4992, 1000, 128, torch.float16, torch.float32),   # whole-stage groups, 39 stages
+    (7, 1920, 130, 384, torch.bfloat16, torch.float16),    # groups of three stages
+    (9, 1920, 130, 96, torch.bfloat16, torch.float16),     # groups that straddle stages
+    (17, 1152, 8200, 32, torch.float16, torch.bfloat16),   # two activation tiles (the second of one row), two weight tiles
+    (32, 2176, 300, 64, torch.bfloat16, torch.float16),    # two activation tiles, one weight tile
+    (50, 896, 2000, 32, torch.bfloat16, torch.float16),    # four activation tiles
+    (70, 14336, 4100, 32, torch.bfloat16, torch.float16),  # a scale table past the untiled kernel's LDS: two blocks of rows
+])
+def test_group_kernel(device, m, k, n, g, act, sdt):
+    """The group kernel (small m with groups of 32 or 64 keys, or stages that the skinny
+    kernel does not split): every tile shape, runs shorter than a round, ragged M and N,
+    random zero points, strided activations. Within the tolerance of the float64 oracle,
+    bit-identical across repeats."""
+    print(f"w4a16 group m={m} k={k} n={n} g={g} {act} {sdt}", flush=True)
+    x, qw, s, z, ref = _host_case(n, k, m, g, seed=m + k + n, act=act, sdt=sdt, zeros="random")
+    xd, qd, sd, zd = x.to(device), qw.to(device), s.to(device), z.to(device)
+    y = w4a16_gemm(xd, qd, sd, zd, g)
+    assert y.dtype == act
+    _assert_close(y, ref, f"group m={m} k={k} n={n} g={g}")
+    assert torch.equal(y, w4a16_gemm(xd, qd, sd, zd, g))
+    xs = torch.zeros(m, k + 72, dtype=act, device=device)[:, 40:40 + k]  # rows 16-byte aligned, stride k + 72
+    xs.copy_(xd)
+    assert torch.equal(w4a16_gemm(xs, qd, sd, zd, g), y)
+
+
 # (plans as the host computes them for 256 CUs: panels of 16 MT rows, 256-row weight tiles)
 @pytest.mark.parametrize("m,k,n,act,sdt", [
     (150, 2048, 20480, torch.float16, torch.bfloat16),   # MT 8, the last panel of 22 rows
