@@ -36,6 +36,7 @@
 //
 // Generic path (any other shape, fp32 activations): one thread per output,
 // fp32 dequant and dot product.
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 
@@ -1821,8 +1822,8 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
     // the panel kernel (weights rounded to the operand type in the same way) where its
     // taller tiles come out ahead. The wide kernel takes 2.15 us a stage and round of one
     // workgroup per CU (m = 197 and 512 x 4096 x 28672: 2.2 us).
-    const int64_t cus = ss_host::device_cu_count();
-    const int64_t rounds = ((int64_t)pl.ks * pl.n_tiles * pl.m_blocks + cus - 1) / cus;
+    const int64_t xcd_cus = std::max(1, ss_host::device_cu_count() / 8);  // whole pairs go to one XCD
+    const int64_t rounds = (((int64_t)pl.ks * pl.n_tiles + 7) / 8 * pl.m_blocks + xcd_cus - 1) / xcd_cus;
     double t = (double)rounds * (2.15 * pl.kchunk * pl.ns / kWideNS + 4.0);
     if (pl.ks > 1) t += (double)pl.ks * (double)m * (double)n * 8e-6 / 4.0 + 4.0;
     if (allow_panel && plan_w4a16_panel(pl.pp, m, n, k, g, t)) {

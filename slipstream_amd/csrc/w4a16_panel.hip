@@ -108,14 +108,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 15, kg = lane >> 4;
-  // workgroup -> (K range, weight tile, activation block): the activation blocks of one
-  // (range, weight tile) pair 8 ids apart, on one XCD, so its L2 serves their weights
-  const int blk = blockIdx.x / (8 * m_blocks), within = blockIdx.x - blk * 8 * m_blocks;
-  const int pair = blk * 8 + (within & 7);
-  if (pair >= ks * n_tiles) return;
+  // workgroup -> (K range, weight tile, activation block): each XCD (workgroups go round
+  // robin over the eight) takes a contiguous eighth of the list, in which the activation
+  // blocks of a (range, weight tile) pair follow each other, so that its L2 serves their
+  // weights and no XCD has more than its share (whole pairs per XCD: 2158 x 2560 x 4864,
+  // 19 pairs of 12 blocks, put 36 workgroups on three of them and took two rounds, 104 us)
+  const int total = ks * n_tiles * m_blocks, per_xcd = (total + 7) >> 3;
+  const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (item >= total) return;
+  const int pair = item / m_blocks;
   const int zr = pair % ks;
   const int nb = (pair / ks) * kPanelRows + wave * 64;  // this wave's weight rows
-  const int m0 = (within >> 3) * BM;
+  const int m0 = (item - pair * m_blocks) * BM;
   const int rows = min(BM, p.m - m0);
   const int i0 = zr * kchunk;
   const int i1 = min(p.k >> 7, i0 + kchunk);
@@ -362,8 +366,7 @@ int launch_panel(const W4Params& p, const PanelPlan& pl, float* part, hipStream_
     }
     attr_set = true;
   }
-  const int64_t pairs = (int64_t)pl.ks * pl.n_tiles;
-  const int64_t grid = (pairs + 7) / 8 * 8 * pl.m_blocks;
+  const int64_t grid = ((int64_t)pl.ks * pl.n_tiles * pl.m_blocks + 7) / 8 * 8;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, stream, p, part, pl.kchunk, pl.ks, pl.n_tiles,
                      pl.m_blocks);
   return ss_host::launch_status("w4a16 gemm (panel)");
@@ -414,7 +417,7 @@ bool plan_w4a16_panel(PanelPlan& pl, int64_t m, int64_t n, int64_t k, int g, dou
     }
   }
   return found && (pl.ks == 1 || (int64_t)pl.ks * m * n * 4 < (int64_t)kOutOfRange) &&
-         ((int64_t)pl.ks * pl.n_tiles + 7) / 8 * 8 * pl.m_blocks <= 0x7fffffff;
+         (int64_t)pl.ks * pl.n_tiles * pl.m_blocks <= 0x7ffffff0;
 }
 
 int launch_w4a16_panel(const W4Params& p, const PanelPlan& pl, int act_dtype, float* part, hipStream_t stream) {
