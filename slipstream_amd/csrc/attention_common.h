@@ -53,8 +53,9 @@ struct AttnParams {
   int chunk_tokens;   // > 0: sequence b is chunk b of a prefix of prefix_tokens keys:
   int prefix_tokens;  //   min(chunk_tokens, prefix_tokens - b * chunk_tokens) keys, no
                       //   ctx_lens, and query tokens [b * q_period, (b + 1) * q_period)
-  int work_qtiles;    // > 0: the prefill takes entry e = (e / work_qtiles, e % work_qtiles)
-                      //   of batch * work_qtiles, in order, instead of a work list
+  int work_qtiles;    // > 0: the prefill takes entry e = sequence e / work_qtiles, query tile
+                      //   work_qtiles - 1 - e % work_qtiles, in order, instead of a work list
+  int split;          // prefill_split_kernel: key parts of an item (ws_o, ws_ml hold the partial rows)
   const void* px_part;  // S normalised prefix parts [S][batch * n_q][D] of the head_dim type
   const float* px_lse;  // and their log2-domain log-sum-exp [S][batch * n_q]
   int px_n;             // S: the decode and its merge fold the parts into every row

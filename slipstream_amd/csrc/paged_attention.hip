@@ -26,7 +26,7 @@ int64_t prefill_work_bytes(int64_t batch, int n_rep, int max_query_len);
 int64_t prefill_row_cap(int n_rep, int max_query_len);
 // planned: work already holds the list (count, then (b << 16) | query tile per entry)
 int launch_prefill(const AttnParams& p, int dtype, int head_dim, int max_query_len, int* work,
-                   int64_t work_bytes, hipStream_t stream, bool planned);
+                   int64_t work_bytes, hipStream_t stream, bool planned, void* ws, int64_t ws_bytes);
 int read_status(int* flags, int clear, hipStream_t stream);
 int64_t general_workspace_bound(int n_q, int n_kv, int head_dim, int max_query_len);
 int launch_general(const AttnParams& p, int dtype, int head_dim, int max_query_len, bool vec, void* ws,
@@ -147,8 +147,9 @@ int run(AttnParams& p, int dtype, int head_dim, int max_query_len, void* workspa
                              plan_qtiles, planned, defer);
   };
   auto prefill = [&](hipStream_t s, bool planned) {
+    // (without decode rows the whole workspace is the prefill's, for a split of its keys)
     return ss::launch_prefill(p, dtype, head_dim, max_query_len, list, has_list ? ws_bytes - dec_bytes : 0, s,
-                              planned);
+                              planned, decode_rows ? nullptr : workspace, decode_rows ? 0 : ws_bytes);
   };
   // A packed step has both kinds of rows. They run one after the other: each kernel
   // fills every CU with one workgroup (registers, LDS), and the split-K decode finishes

@@ -253,6 +253,69 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   prefill_tile_body<T, D>(p, work, blockIdx.x, gridDim.x);
 }
 
+// A prefill with fewer items than CUs (a chunk alone: 256 tokens of a 32/8-head model are 64
+// items) leaves most of the chip idle and its few workgroups walk the keys alone: the keys
+// of every item are split over workgroups (prefill_split_kernel), fp32 partial rows and
+// their (max, sum) go to the workspace, and prefill_split_merge_kernel adds them.
+template <typename T, int D>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_split_kernel(
+    const AttnParams p) {
+  prefill_tile_body<T, D, true>(p, nullptr, blockIdx.x, gridDim.x);
+}
+
+// One thread per four outputs of a row: the parts' rows weighted by 2^(m - max), all loads
+// of four parts in flight, divided by the weighted sum.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void prefill_split_merge_kernel(const AttnParams p) {
+  constexpr int TPR = D / 4;  // threads of a row
+  const int64_t r = ((int64_t)blockIdx.x * 256 + threadIdx.x) / TPR;
+  const int d = 4 * (threadIdx.x % TPR);
+  const int item = (int)(r >> 7), row = (int)(r & 127);
+  const int entry = item / p.n_kv, h = item - entry * p.n_kv;
+  const int b = entry / p.work_qtiles, qt = p.work_qtiles - 1 - (entry - b * p.work_qtiles);
+  const int rr = qt * 128 + row;
+  if (b >= p.batch || rr >= p.tq * p.n_rep) return;
+  const int64_t base = ((int64_t)item * p.split) * 128 + row;
+  float mx = kNegBig;
+  for (int i = 0; i < p.split; ++i) mx = fmaxf(mx, p.ws_ml[2 * (base + 128 * i)]);
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+  for (int i0 = 0; i0 < p.split; i0 += 4) {
+    f32x4 x[4];
+    float2 ml[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t at = base + 128 * min(i0 + i, p.split - 1);
+      ml[i] = *reinterpret_cast<const float2*>(p.ws_ml + 2 * at);
+      x[i] = *reinterpret_cast<const f32x4*>(p.ws_o + at * D + d);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float w = i0 + i < p.split && ml[i].y > 0.f ? fast_exp2(ml[i].x - mx) : 0.f;
+      l = fmaf(w, ml[i].y, l);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = fmaf(w, x[i][e], o[e]);
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int j = rr / p.n_rep, hq = h * p.n_rep + (rr - j * p.n_rep);
+  T* const out = (T*)p.out + (int64_t)b * p.o_sb + (int64_t)j * p.o_st + (int64_t)hq * p.o_sh + d;
+  *reinterpret_cast<u32x2*>(out) = u32x2{Elem<T>::pack2(o[0] * inv, o[1] * inv), Elem<T>::pack2(o[2] * inv, o[3] * inv)};
+}
+
+// Key parts per item of a padded prefill: as many as keep one workgroup per CU, of at least
+// three 64-key tiles of the widest table, within the workspace; 1: not split. Where two
+// parts just fit it still pays (512 tokens over 2000, 128 items: 58.5 -> 42.4 us).
+int prefill_split(const AttnParams& p, int64_t items, int head_dim, int64_t ws_bytes) {
+  const int64_t tiles = (((int64_t)p.max_blocks << p.bs_shift) + 63) / 64;
+  int64_t s = ss_host::device_cu_count() / items;
+  s = s < tiles / 3 ? s : tiles / 3;
+  s = s < 16 ? s : 16;
+  const int64_t part = items * 128 * (head_dim + 2) * 4;
+  while (s > 1 && s * part > ws_bytes) --s;
+  return s < 1 ? 1 : (int)s;
+}
+
 // The tiled prefill's work list (plan_work_list) built by a one-workgroup launch, when
 // no decode launch of the same call builds it.
 __global__ __launch_bounds__(1024) void prefill_plan_kernel(const AttnParams p, int* __restrict__ work,
@@ -264,7 +327,7 @@ constexpr int kPrefillNT = 2;
 
 template <typename T, int D>
 int launch_prefill_typed(const AttnParams& p, int max_query_len, int* work, int64_t work_bytes, bool planned,
-                         hipStream_t stream) {
+                         void* ws, int64_t ws_bytes, hipStream_t stream) {
   if (D <= 128 && p.block_size >= 16) {
     constexpr int rows = 128;
     const int64_t qtiles = ((int64_t)max_query_len * p.n_rep + rows - 1) / rows;
@@ -273,6 +336,35 @@ int launch_prefill_typed(const AttnParams& p, int max_query_len, int* work, int6
       ss_host::set_error("paged attention prefill: too many query tiles (%lld per sequence, batch %d)",
                          (long long)qtiles, p.batch);
       return SS_ERR_UNSUPPORTED;
+    }
+    constexpr int DD = D <= 128 ? D : 128;
+    const int lds = 6 * TileCfg<T, DD>::PLANE;
+    const int64_t items = (int64_t)p.batch * qtiles * p.n_kv;
+    // (padded calls only: every sequence has the same query tiles, so all parts are written)
+    const int split = ws && ((uintptr_t)ws & 15) == 0 && !p.cu && !p.lse && p.chunk_tokens == 0 && p.work_qtiles == 0 && !planned && !p.noncausal
+                          ? prefill_split(p, items, DD, ws_bytes)
+                          : 1;
+    if (split > 1) {
+      static bool split_attr_set = false;  // per instantiation; the attribute is process-wide
+      if (!split_attr_set) {
+        if (hipFuncSetAttribute((const void*)prefill_split_kernel<T, DD>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                lds) != hipSuccess) {
+          ss_host::set_error("paged attention prefill: cannot reserve %d bytes of LDS", lds);
+          return SS_ERR_UNSUPPORTED;
+        }
+        split_attr_set = true;
+      }
+      AttnParams ps = p;
+      ps.split = split;
+      ps.work_qtiles = (int)qtiles;
+      ps.ws_o = (float*)ws;
+      ps.ws_ml = (float*)ws + items * split * 128 * DD;
+      hipLaunchKernelGGL((prefill_split_kernel<T, DD>), dim3((unsigned)(items * split)), dim3(512), lds, stream, ps);
+      int st = ss_host::launch_status("paged attention prefill (split)");
+      if (st != SS_OK) return st;
+      hipLaunchKernelGGL((prefill_split_merge_kernel<T, DD>), dim3((unsigned)(items * 128 * (DD / 4) / 256)), dim3(256),
+                         0, stream, ps);
+      return ss_host::launch_status("paged attention prefill merge");
     }
     const int64_t need = p.work_qtiles > 0 ? 0 : prefill_work_bytes(p.batch, p.n_rep, max_query_len);
     if (p.work_qtiles > 0 && p.work_qtiles != qtiles) {
@@ -285,8 +377,6 @@ int launch_prefill_typed(const AttnParams& p, int max_query_len, int* work, int6
                          (long long)work_bytes, (long long)need);
       return SS_ERR_WORKSPACE;
     }
-    constexpr int DD = D <= 128 ? D : 128;
-    const int lds = 6 * TileCfg<T, DD>::PLANE;
     static bool attr_set = false;  // per instantiation; the attribute is process-wide
     if (!attr_set) {
       if (hipFuncSetAttribute((const void*)prefill_tile_kernel<T, DD>,
@@ -296,16 +386,19 @@ int launch_prefill_typed(const AttnParams& p, int max_query_len, int* work, int6
       }
       attr_set = true;
     }
-    if (!planned && p.work_qtiles == 0) {
+    // One sequence needs no list: its tiles from the last down are already costliest first
+    // (the plan's launch and the gap after it took about 6 us)
+    AttnParams pp = p;
+    if (!planned && p.work_qtiles == 0 && !p.cu && p.batch == 1) pp.work_qtiles = (int)qtiles;
+    if (!planned && pp.work_qtiles == 0) {
       hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(kPlanBuckets), 0, stream, p, work, (int)qtiles);
       int st = ss_host::launch_status("paged attention prefill plan");
       if (st != SS_OK) return st;
     }
     // one resident workgroup per CU (the LDS rings take 96 KB); never more than items
-    const int64_t items = (int64_t)p.batch * qtiles * p.n_kv;
     const int64_t cus = ss_host::device_cu_count();
     const int grid = (int)(items < cus ? items : cus);
-    hipLaunchKernelGGL((prefill_tile_kernel<T, DD>), dim3((unsigned)grid), dim3(512), lds, stream, p,
+    hipLaunchKernelGGL((prefill_tile_kernel<T, DD>), dim3((unsigned)grid), dim3(512), lds, stream, pp,
                        (const int*)work);
     return ss_host::launch_status("paged attention prefill");
   }
@@ -340,15 +433,15 @@ int64_t prefill_work_bytes(int64_t batch, int n_rep, int max_query_len) {
 }
 
 int launch_prefill(const AttnParams& p, int dtype, int head_dim, int max_query_len, int* work,
-                   int64_t work_bytes, hipStream_t stream, bool planned) {
+                   int64_t work_bytes, hipStream_t stream, bool planned, void* ws, int64_t ws_bytes) {
   if (dtype == SS_DTYPE_BF16) {
-    if (head_dim == 64) return launch_prefill_typed<bf16_t, 64>(p, max_query_len, work, work_bytes, planned, stream);
-    if (head_dim == 128) return launch_prefill_typed<bf16_t, 128>(p, max_query_len, work, work_bytes, planned, stream);
-    return launch_prefill_typed<bf16_t, 256>(p, max_query_len, work, work_bytes, planned, stream);
+    if (head_dim == 64) return launch_prefill_typed<bf16_t, 64>(p, max_query_len, work, work_bytes, planned, ws, ws_bytes, stream);
+    if (head_dim == 128) return launch_prefill_typed<bf16_t, 128>(p, max_query_len, work, work_bytes, planned, ws, ws_bytes, stream);
+    return launch_prefill_typed<bf16_t, 256>(p, max_query_len, work, work_bytes, planned, ws, ws_bytes, stream);
   }
-  if (head_dim == 64) return launch_prefill_typed<f16_t, 64>(p, max_query_len, work, work_bytes, planned, stream);
-  if (head_dim == 128) return launch_prefill_typed<f16_t, 128>(p, max_query_len, work, work_bytes, planned, stream);
-  return launch_prefill_typed<f16_t, 256>(p, max_query_len, work, work_bytes, planned, stream);
+  if (head_dim == 64) return launch_prefill_typed<f16_t, 64>(p, max_query_len, work, work_bytes, planned, ws, ws_bytes, stream);
+  if (head_dim == 128) return launch_prefill_typed<f16_t, 128>(p, max_query_len, work, work_bytes, planned, ws, ws_bytes, stream);
+  return launch_prefill_typed<f16_t, 256>(p, max_query_len, work, work_bytes, planned, ws, ws_bytes, stream);
 }
 
 }  // namespace ss

@@ -123,7 +123,10 @@ extern __shared__ __attribute__((aligned(1024))) char s_tile_stages[];
 // for the occupancy that size alone allows.
 // The body of prefill_tile_kernel as workgroup wg of G (the shared-prefix cascade runs
 // it in the first G workgroups of a launch whose others run the decode).
-template <typename T, int D>
+// SPLIT: the keys of every item in p.split contiguous parts of 64-key tiles, one workgroup
+// each (all entries in order, no list): fp32 partial rows into p.ws_o and their (max, sum)
+// into p.ws_ml, which prefill_split_merge_kernel combines.
+template <typename T, int D, bool SPLIT = false>
 __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int* __restrict__ work, const int wg,
                                                   const int G) {
   typedef TileCfg<T, D> C;
@@ -141,15 +144,16 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
   // e * n_kv + h, one per KV head) in snake order: round r takes item r*G + j, or
   // r*G + G-1-j in odd rounds, so a workgroup that drew a long item early draws a
   // short one next.
-  // (With p.work_qtiles > 0 the entries are every (sequence, tile) in order, equal in
-  // cost up to the last sequence's, and no list is read.)
+  // (With p.work_qtiles > 0 no list is read: the entries are every (sequence, tile), the
+  // sequences in order and each one's tiles from the last, the costliest, down.)
   const int wq = p.work_qtiles;
-  const int total = (wq > 0 ? p.batch * wq : __builtin_amdgcn_readfirstlane(work[0])) * p.n_kv;
+  const int total = (wq > 0 ? p.batch * wq : __builtin_amdgcn_readfirstlane(work[0])) * p.n_kv * (SPLIT ? p.split : 1);
   for (int round = 0; round * G < total; ++round) {
-    const int idx = round * G + ((round & 1) ? G - 1 - wg : wg);
-    if (idx >= total) continue;
+    const int slot = round * G + ((round & 1) ? G - 1 - wg : wg);
+    if (slot >= total) continue;
+    const int idx = SPLIT ? slot / p.split : slot, part = SPLIT ? slot - idx * p.split : 0;
     const int entry = idx / p.n_kv;
-    const int bq = wq > 0 ? ((entry / wq) << 16) | (entry % wq) : __builtin_amdgcn_readfirstlane(work[1 + entry]);
+    const int bq = wq > 0 ? ((entry / wq) << 16) | (wq - 1 - entry % wq) : __builtin_amdgcn_readfirstlane(work[1 + entry]);
     [&](const int b, const int qt, const int h) {
   int qlen;
   int64_t qoff;
@@ -170,8 +174,13 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
   const int ctx = __builtin_amdgcn_readfirstlane(kv_len(p, b));
   const int kvt = seq_kv_tokens(p, ctx);
   const int last_row = min(R - 1, row0 + ROWS - 1);
-  const int kv_end = p.noncausal ? kvt : min(kvt, ctx - qlen + last_row / p.n_rep + 1);
-  const int ntiles = kv_end > 0 ? (kv_end + C::KT - 1) / C::KT : 0;
+  const int kv_all = p.noncausal ? kvt : min(kvt, ctx - qlen + last_row / p.n_rep + 1);
+  const int tiles_all = kv_all > 0 ? (kv_all + C::KT - 1) / C::KT : 0;
+  // this workgroup's tiles [t0, ntiles): all of them, or its part
+  const int per_part = SPLIT ? (tiles_all + p.split - 1) / p.split : tiles_all;
+  const int t0 = SPLIT ? part * per_part : 0;
+  const int ntiles = SPLIT ? min(tiles_all, t0 + per_part) : tiles_all;
+  const int kv_end = SPLIT ? min(kv_all, ntiles * C::KT) : kv_all;
   const ConstTable table = (ConstTable)(p.bt + (int64_t)b * p.bt_stride);
 
   // query rows of this lane (column n of row tile nt) and their causal limits;
@@ -423,7 +432,7 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
   // group's entry per tile and no tile needs validity bits.
   const bool k_loader = wave < 4, v_loader = wave >= 4;
   bool bad = false;
-  for (int i = threadIdx.x; i * p.block_size < kv_end; i += 512) {
+  for (int i = ((t0 * C::KT) >> p.bs_shift) + threadIdx.x; i * p.block_size < kv_end; i += 512) {
     const int v = p.bt[(int64_t)b * p.bt_stride + i];
     bad |= v < 0 || v >= p.num_blocks;
   }
@@ -449,18 +458,18 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
       }
     };
     int ph0, ph1, ph2, vb0, vb1, vb2;
-    fetch(0);
-    tile_info(0, ph0, vb0);
-    if (k_loader) issue(0, ph0, kplane, kring);
-    fetch(1);
-    tile_info(1, ph1, vb1);
-    if (k_loader) issue(1, ph1, kplane, kring + C::PLANE);
-    if (v_loader) issue(0, ph0, vplane, vring);
-    fetch(2);
-    tile_info(2, ph2, vb2);
-    if (k_loader) issue(2, ph2, kplane, kring + 2 * C::PLANE);
-    if (v_loader) issue(1, ph1, vplane, vring + C::PLANE);
-    fetch(3);
+    fetch(t0);
+    tile_info(t0, ph0, vb0);
+    if (k_loader) issue(t0, ph0, kplane, kring);
+    fetch(t0 + 1);
+    tile_info(t0 + 1, ph1, vb1);
+    if (k_loader) issue(t0 + 1, ph1, kplane, kring + C::PLANE);
+    if (v_loader) issue(t0, ph0, vplane, vring);
+    fetch(t0 + 2);
+    tile_info(t0 + 2, ph2, vb2);
+    if (k_loader) issue(t0 + 2, ph2, kplane, kring + 2 * C::PLANE);
+    if (v_loader) issue(t0 + 1, ph1, vplane, vring + C::PLANE);
+    fetch(t0 + 3);
     // three score buffers, one per unrolled step: tile t's scores live in s[t % 3]
     f32x4 sa[NT][XS], sb[NT][XS], sc[NT][XS];
     // group 0 landed; groups 1 and 2 may be in flight (a V loader's first load is
@@ -479,7 +488,7 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
       fetch(t + 4);
       tile_step(t, vcur, (r + 1) % 3, scur, snext, r);
     };
-    for (int t = 0; t < ntiles; t += 3) {
+    for (int t = t0; t < ntiles; t += 3) {
       step(t, 0, ph0, vb0, ph2, sa, sb);
       if (t + 1 >= ntiles) break;
       step(t + 1, 1, ph1, vb1, ph0, sb, sc);
@@ -502,7 +511,13 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
   for (int nt = 0; nt < NT; ++nt) {
     const float lt = lsum[nt][0];
     const int rr = row0 + wave * 16 * NT + 16 * nt + n;
-    if (rr < R) {
+    if constexpr (SPLIT) {
+      const int64_t prow = (int64_t)slot * ROWS + (rr - row0);
+      if (g == 0) *reinterpret_cast<float2*>(p.ws_ml + 2 * prow) = float2{mrow[nt], lt};
+      float* const o = p.ws_o + prow * D + (D / 4) * g;
+#pragma unroll
+      for (int w = 0; w < C::DT; ++w) *reinterpret_cast<f32x4*>(o + 4 * (w ^ (g & 1))) = acc[nt][w];
+    } else if (rr < R) {
       const int j = rr / p.n_rep;
       const int hq = h * p.n_rep + (rr - j * p.n_rep);
       const float inv = lt > 0.f ? 1.f / lt : 0.f;

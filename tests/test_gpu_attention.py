@@ -398,6 +398,37 @@ def test_prefill_every_key_weighted(device, ctx, holes):
     assert_attn_close(out, ref, f"prefill bucket weights ctx={ctx} holes={holes}")
 
 
+@pytest.mark.parametrize("heads,dtype,tq,ctx,width,bs", [
+    ((32, 8, 128), torch.bfloat16, 256, [2033], None, 16),         # 64 items in four parts of eight or nine tiles
+    ((32, 8, 128), torch.bfloat16, 5, [1000], None, 16),           # eight items of one tile row, five parts
+    ((14, 2, 64), torch.float16, 131, [1500], 400, 16),            # a table far wider than the context: empty parts
+    ((28, 4, 128), torch.float16, 40, [40, 900, 333], None, 32),   # contexts of one and of fifteen tiles, causal ends inside parts
+    ((32, 8, 128), torch.bfloat16, 100, [20, 800], None, 16),      # rows without a visible key
+])
+def test_prefill_split_keys(device, heads, dtype, tq, ctx, width, bs):
+    """Small padded prefills split the keys of an item over workgroups: parts that end inside
+    a tile's causal edge, empty parts, ragged row tiles, rows with no key, table holes.
+    Against the float64 oracle, and bit-identical across repeats."""
+    n_q, n_kv, d = heads
+    print(f"prefill split {heads} {dtype} tq={tq} ctx={ctx}", flush=True)
+    b = workloads.build_batch(ctx, [tq] * len(ctx), n_q=n_q, n_kv=n_kv, head_dim=d, block_size=bs, dtype=dtype,
+                              device="cpu", seed=tq + sum(ctx))
+    tables = [list(t) for t in b.tables_host]
+    tables[-1][len(tables[-1]) // 2] = -1
+    width = width or b.block_tables.shape[1]
+    bt = torch.full((len(ctx), width), -1, dtype=torch.int32)
+    for i, t in enumerate(tables):
+        bt[i, : len(t)] = torch.tensor(t, dtype=torch.int32)
+    b.block_tables = bt
+    ref = ora.paged_attention(f64(b.padded_q()), f64(b.kv_cache), tables_array(tables, width), np.array(b.ctx_host), 0,
+                              b.scale, bs)
+    _to(b, device)
+    out = paged_attention_prefill(b.padded_q(), b.kv_cache, b.block_tables, b.context_lens, 0, b.scale, bs)
+    assert_attn_close(out, ref, f"prefill split tq={tq} ctx={ctx}")
+    again = paged_attention_prefill(b.padded_q(), b.kv_cache, b.block_tables, b.context_lens, 0, b.scale, bs)
+    assert torch.equal(out, again)
+
+
 def test_prefill_head_dim_256(device):
     b = workloads.build_batch([40, 300], [40, 40], n_q=8, n_kv=2, head_dim=256, block_size=16,
                               dtype=torch.bfloat16, device="cpu", seed=256)
