@@ -19,7 +19,7 @@ struct W4Params {
 
 // The panel kernel (w4a16_panel.hip): its grid and K split.
 struct PanelPlan {
-  int mt;  // 16-row activation tiles of a workgroup
+  int mt, ns;  // 16-row activation tiles of a workgroup, 16-row weight tiles of a wave
   int ks, kchunk;  // K ranges and 128-key stages per range
   int n_tiles, m_blocks;
 };

@@ -2,13 +2,15 @@
 // cores, not the weight bytes, set the time (a prefill chunk's or a packed step's tokens).
 //
 // A workgroup of four waves, one per SIMD, multiplies a panel of 16 MT activation rows
-// (MT = 8 to 16) with 256 weight rows; wave w owns 64 of them (four 16-row MFMA tiles)
+// (MT = 8 to 16) with 64 NS weight rows; wave w owns 16 NS of them (NS = 4 16-row MFMA tiles,
+// or two where m fits one panel and 256-row tiles would leave half the chip idle: 197 x
+// 4096 x 28672 73.6 -> 66.4 us, 130 x 4096 x 28672 73.7 -> 54.0)
 // against every activation row of the panel. Per 128-key stage (one quantisation group):
 //   - every weight is unpacked and dequantised once per workgroup, straight into the MFMA
 //     operand registers (19 VALU instructions per eight weights), and feeds MT MFMAs: at
 //     MT = 16 1.2 VALU instructions per MFMA, which issue while the matrix core works;
-//   - every activation fragment read from LDS feeds four MFMAs (the wide kernel's two make
-//     its LDS reads as long as its MFMAs).
+//   - every activation fragment read from LDS feeds NS MFMAs (the wide kernel's two, with
+//     eight waves reading, make its LDS reads as long as its MFMAs).
 // Activations come into LDS by DMA in half stages of 64 keys, a ring of four: one being
 // read, one landed (so that fragments are read ahead across the barrier), two on their
 // way. One wave per SIMD has nothing to hide behind, so the order is written out: every
@@ -17,8 +19,8 @@
 // stages ahead), and the scheduler is held to that order.
 //
 // The weights are the MFMA's row operand, so a lane's accumulators are consecutive output
-// columns; with tile row i of wave tile ns holding weight row 16 (i / 4) + 4 ns + i % 4 they
-// are sixteen consecutive ones, stored as they are (no pass through LDS).
+// columns; with tile row i of wave tile ns holding weight row 4 NS (i / 4) + 4 ns + i % 4 they
+// are 4 NS consecutive ones, stored as they are (no pass through LDS).
 //
 // Measured: 2240 x 4096 x 28672 662 -> 444 us (794 -> 1184 TFLOP/s; the dense bf16 product
 // through hipBLASLt 365 us on the same card, these MFMAs alone with no loads or
@@ -32,7 +34,6 @@
 namespace ss {
 namespace {
 
-constexpr int kPanelRows = 256;  // weight rows of a workgroup
 constexpr int kPanelTab = 4 * 2 * 64 * 8;  // LDS bytes of the four waves' scale tables (two stages each)
 
 // Eight int4 weights (one word: keys 8j .. 8j + 7 of a row) -> T((q - z) s) in key order.
@@ -95,10 +96,10 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-template <typename T, int MT>
+template <typename T, int MT, int NS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void w4a16_panel_kernel(
     const W4Params p, float* __restrict__ part, int kchunk, int ks, int n_tiles, int m_blocks) {
-  constexpr int NS = 4;
+  constexpr int WR = 16 * NS;  // weight rows of a wave
   constexpr int BM = 16 * MT;
   constexpr int XBYTES = BM * 128;  // one half stage of activations (64 keys)
   constexpr int XI = MT / 2;        // DMA instructions per wave and half stage (eight rows each)
@@ -118,19 +119,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   if (item >= total) return;
   const int pair = item / m_blocks;
   const int zr = pair % ks;
-  const int nb = (pair / ks) * kPanelRows + wave * 64;  // this wave's weight rows
+  const int nb = (pair / ks) * 4 * WR + wave * WR;  // this wave's weight rows
   const int m0 = (item - pair * m_blocks) * BM;
   const int rows = min(BM, p.m - m0);
   const int i0 = zr * kchunk;
   const int i1 = min(p.k >> 7, i0 + kchunk);
-  float2* const s_tab = reinterpret_cast<float2*>(s_dyn + 4 * XBYTES) + wave * 128;  // [stage % 2][64 rows]
+  float2* const s_tab = reinterpret_cast<float2*>(s_dyn + 4 * XBYTES) + wave * 2 * WR;  // [stage % 2][WR rows]
 
   // ---- weights: tile ns is 4 ns rows further on; rows past N read zeros (out of the
   // descriptor's range, no memory access) and are never stored. Half h of a stage: keys
   // 64 h + 16 kg .. + 15 of the lane's row, its key steps' words 0 and 1.
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(p.qw, (uint32_t)((int64_t)p.n * p.k / 2));
   const int w_row = p.k / 2;  // bytes
-  const int w_off = (nb + (ln >> 2) * 16 + (ln & 3)) * w_row + 8 * kg;
+  const int w_off = (nb + (ln >> 2) * 4 * NS + (ln & 3)) * w_row + 8 * kg;
   typedef u32x2 Words[NS][2];
   auto load_w1 = [&](int i, int ns, int h, Words& w) {
     w[ns][h] = __builtin_bit_cast(
@@ -143,12 +144,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       for (int h = 0; h < 2; ++h) load_w1(i, ns, h, w);
   };
 
-  // ---- scale and zero point of the wave's 64 rows at one stage, one row per lane, turned
+  // ---- scale and zero point of the wave's rows at one stage, one row per lane, turned
   // around through the wave's own table
   const int esize = p.sdt == SS_DTYPE_F32 ? 4 : 2;
   const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(p.sc, (uint32_t)((int64_t)p.n * p.groups * esize));
   const __amdgpu_buffer_rsrc_t rzp = buffer_rsrc(p.qz, (uint32_t)((int64_t)p.n * p.groups * 4));
-  const int g_row = min(nb + lane, p.n - 1) * p.groups;
+  const int g_row = min(nb + lane % WR, p.n - 1) * p.groups;
   const uint32_t f16_mask = p.sdt == SS_DTYPE_F16 ? ~0u : 0u, bf16_mask = p.sdt == SS_DTYPE_BF16 ? ~0u : 0u;
   auto load_sz = [&](int i, uint32_t& sb, int& zb) {
     sb = scale_bits(rsc, g_row + i, esize);
@@ -157,10 +158,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   float sc[NS], cz[NS], scn[NS], czn[NS];  // this stage's scales and - s (1024 + z), and the next's
   auto turn_sz = [&](int i, uint32_t sb, int zb) {
     const float s = decode_scale_masked(sb, f16_mask, bf16_mask);
-    s_tab[(i & 1) * 64 + lane] = float2{s, -s * (1024.f + (float)zb)};
+    s_tab[(i & 1) * WR + lane % WR] = float2{s, -s * (1024.f + (float)zb)};
 #pragma unroll
     for (int ns = 0; ns < NS; ++ns) {
-      const float2 t = s_tab[(i & 1) * 64 + (ln >> 2) * 16 + ns * 4 + (ln & 3)];
+      const float2 t = s_tab[(i & 1) * WR + (ln >> 2) * 4 * NS + ns * 4 + (ln & 3)];
       scn[ns] = t.x;
       czn[ns] = t.y;
     }
@@ -305,10 +306,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     for (int ns = 0; ns < NS; ++ns) asm volatile("" : "+a"(acc[mt][ns]));
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA into LDS is left when the workgroup ends
 
-  // ---- results: lane holds C[m0 + 16 mt + ln][nb + 16 kg + 4 ns + e]
-  const int n = nb + 16 * kg;
+  // ---- results: lane holds C[m0 + 16 mt + ln][nb + 4 NS kg + 4 ns + e]
+  const int n = nb + 4 * NS * kg;
   if (n >= p.n) return;
-  const bool whole = n + 16 <= p.n;
+  const bool whole = n + 4 * NS <= p.n;
   if (ks > 1) {
     const bool vec = whole && p.n % 4 == 0;
 #pragma unroll
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     T* const o = (T*)p.out + (int64_t)m * p.o_stride + n;
     if (vec) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < NS / 2; ++h)
         store16(o + 8 * h, u32x4{Elem<T>::pack2(acc[mt][2 * h][0], acc[mt][2 * h][1]),
                                  Elem<T>::pack2(acc[mt][2 * h][2], acc[mt][2 * h][3]),
                                  Elem<T>::pack2(acc[mt][2 * h + 1][0], acc[mt][2 * h + 1][1]),
@@ -354,9 +355,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
 size_t panel_lds_bytes(int mt) { return (size_t)4 * mt * 16 * 128 + kPanelTab; }
 
-template <typename T, int MT>
+template <typename T, int MT, int NS>
 int launch_panel(const W4Params& p, const PanelPlan& pl, float* part, hipStream_t stream) {
-  auto kern = w4a16_panel_kernel<T, MT>;
+  auto kern = w4a16_panel_kernel<T, MT, NS>;
   static bool attr_set = false;
   const size_t lds = panel_lds_bytes(MT);
   if (!attr_set) {
@@ -374,12 +375,22 @@ int launch_panel(const W4Params& p, const PanelPlan& pl, float* part, hipStream_
 
 template <typename T>
 int launch_panel_typed(const W4Params& p, const PanelPlan& pl, float* part, hipStream_t stream) {
-  switch (pl.mt) {
-    case 8: return launch_panel<T, 8>(p, pl, part, stream);
-    case 10: return launch_panel<T, 10>(p, pl, part, stream);
-    case 12: return launch_panel<T, 12>(p, pl, part, stream);
-    case 14: return launch_panel<T, 14>(p, pl, part, stream);
-    case 16: return launch_panel<T, 16>(p, pl, part, stream);
+  if (pl.ns == 4) {
+    switch (pl.mt) {
+      case 8: return launch_panel<T, 8, 4>(p, pl, part, stream);
+      case 10: return launch_panel<T, 10, 4>(p, pl, part, stream);
+      case 12: return launch_panel<T, 12, 4>(p, pl, part, stream);
+      case 14: return launch_panel<T, 14, 4>(p, pl, part, stream);
+      case 16: return launch_panel<T, 16, 4>(p, pl, part, stream);
+    }
+  } else {
+    switch (pl.mt) {
+      case 8: return launch_panel<T, 8, 2>(p, pl, part, stream);
+      case 10: return launch_panel<T, 10, 2>(p, pl, part, stream);
+      case 12: return launch_panel<T, 12, 2>(p, pl, part, stream);
+      case 14: return launch_panel<T, 14, 2>(p, pl, part, stream);
+      case 16: return launch_panel<T, 16, 2>(p, pl, part, stream);
+    }
   }
   ss_host::set_error("w4a16 gemm: panel of %d tiles", pl.mt);
   return SS_ERR_UNSUPPORTED;
@@ -389,26 +400,31 @@ int launch_panel_typed(const W4Params& p, const PanelPlan& pl, float* part, hipS
 
 // The panel height and K split of least estimated time, and whether that beats a kernel
 // of estimated time `other` (us). A workgroup takes 0.95 + 0.143 MT us a stage (MT = 8: 2.07
-// us, 16: 3.25 us measured, one workgroup per CU) and about 4 us around its stages; a K
-// split adds the partials' round trip (4 TB/s) and the reduce launch.
+// us, 16: 3.25 us measured, one workgroup per CU), with two weight tiles a wave 1.0 + 0.068
+// MT (MT = 10: 1.6, 16: 2.15), and about 4 us around its stages; a K split adds the partials'
+// round trip (4 TB/s) and the reduce launch. The constant part is the dequantisation's and
+// the loads' issue: one wave issues an instruction every five cycles or so.
 bool plan_w4a16_panel(PanelPlan& pl, int64_t m, int64_t n, int64_t k, int g, double other) {
-  if (m <= 64 || g != 128 || k % 128 || (n + kPanelRows) * (k / 2) >= ((int64_t)1 << 31)) return false;
-  const int64_t stages = k / 128, n_tiles = (n + kPanelRows - 1) / kPanelRows;
+  if (m <= 64 || g != 128 || k % 128 || (n + 256) * (k / 2) >= ((int64_t)1 << 31)) return false;
+  const int64_t stages = k / 128;
   const int64_t cus = ss_host::device_cu_count();
   double best = 0.93 * other;  // within the estimate's error the other kernel keeps the shape
   bool found = false;
-  for (int mt : {8, 10, 12, 14, 16}) {
+  for (int shape = 0; shape < 10; ++shape) {
+    const int ns = shape < 5 ? 4 : 2, mt = 8 + 2 * (shape % 5);
+    const int64_t n_tiles = (n + 64 * ns - 1) / (64 * ns);
     const int64_t m_blocks = (m + 16 * mt - 1) / (16 * mt);
     for (int64_t ks = 1; ks <= 16; ++ks) {
       const int64_t per = (stages + ks - 1) / ks;
       if ((stages + per - 1) / per != ks || (ks > 1 && per < 8)) continue;
       const int64_t rounds = (n_tiles * m_blocks * ks + cus - 1) / cus;
-      double t = (double)rounds * ((double)per * (0.95 + 0.143 * mt) + 4.0);
+      double t = (double)rounds * ((double)per * (ns == 4 ? 0.95 + 0.143 * mt : 1.0 + 0.068 * mt) + 4.0);
       if (ks > 1) t += (double)ks * (double)m * (double)n * 8e-6 / 4.0 + 4.0;
       if (t < best) {
         best = t;
         found = true;
         pl.mt = mt;
+        pl.ns = ns;
         pl.ks = (int)ks;
         pl.kchunk = (int)per;
         pl.n_tiles = (int)n_tiles;

@@ -268,17 +268,23 @@ def test_group_kernel(device, m, k, n, g, act, sdt):
     assert torch.equal(w4a16_gemm(xs, qd, sd, zd, g), y)
 
 
-# (plans as the host computes them for 256 CUs: panels of 16 MT rows, 256-row weight tiles)
+# (plans as the host computes them for 256 CUs: panels of 16 MT rows, 256- or 128-row weight tiles)
 @pytest.mark.parametrize("m,k,n,act,sdt", [
-    (150, 2048, 20480, torch.float16, torch.bfloat16),   # MT 8, the last panel of 22 rows
-    (420, 2048, 20480, torch.bfloat16, torch.float16),   # MT 10, the last panel of 100 rows
-    (520, 2048, 20480, torch.bfloat16, torch.bfloat16),  # MT 12
-    (600, 2048, 20490, torch.float16, torch.float16),    # MT 14, the last weight tile of 10 rows
-    (500, 2048, 28600, torch.bfloat16, torch.float16),   # MT 16, N % 256 = 184
-    (150, 8192, 4100, torch.bfloat16, torch.float16),    # eight K ranges of 8 stages, a weight tile of 4 rows
-    (180, 4096, 8200, torch.bfloat16, torch.float16),    # three K ranges of 11, 11 and 10 stages
-    (600, 4096, 8190, torch.bfloat16, torch.float16),    # two K ranges, N % 4 != 0: element stores of the partials
-    (513, 2048, 16002, torch.bfloat16, torch.float16),   # N % 8 != 0: element stores of the results, one row in the last panel
+    # four weight tiles a wave
+    (300, 2048, 20484, torch.float16, torch.bfloat16),   # MT 8, the last panel of 44 rows, the last weight tile of 4
+    (513, 2048, 16002, torch.bfloat16, torch.float16),   # MT 10, one row in the last panel, N % 8 != 0: element stores
+    (330, 2048, 22532, torch.bfloat16, torch.bfloat16),  # MT 12
+    (420, 2048, 22532, torch.float16, torch.float16),    # MT 14
+    (700, 2048, 16388, torch.bfloat16, torch.float16),   # MT 16
+    (70, 4096, 16388, torch.bfloat16, torch.float16),    # MT 8, three K ranges of 11, 11 and 10 stages
+    # two
+    (300, 2048, 10244, torch.bfloat16, torch.float16),   # MT 8
+    (130, 2048, 16388, torch.float16, torch.float16),    # MT 10
+    (180, 2048, 16388, torch.bfloat16, torch.bfloat16),  # MT 12
+    (200, 2048, 16390, torch.bfloat16, torch.float16),   # MT 14, N % 4 != 0
+    (230, 2048, 16388, torch.float16, torch.bfloat16),   # MT 16
+    (150, 8192, 4100, torch.bfloat16, torch.float16),    # MT 10, seven K ranges of 10 stages, the last of 4
+    (600, 4096, 3074, torch.bfloat16, torch.float16),    # MT 8, two K ranges, N % 4 != 0: element stores of the partials
     (420, 2048, 20480, torch.bfloat16, torch.float32),   # fp32 scales: the wide kernel
 ])
 def test_panel_kernel(device, m, k, n, act, sdt):
