@@ -69,6 +69,21 @@ def test_swiglu_matches_eager(device, dtype, shape):
     _close_within_one_ulp(fused_swiglu(gate, up), F.silu(gate) * up, f"swiglu {shape} {dtype}")
 
 
+@pytest.mark.parametrize("with_residual", [False, True])
+@pytest.mark.parametrize("pieces", [1, 255, 256, 257, 511, 513, 1023, 1025, 2047, 2048])
+def test_rmsnorm_piece_counts(device, pieces, with_residual):
+    """Rows of one 16-byte piece up to the most the threads hold, either side of each count
+    of pieces per thread: threads past the row's end add nothing and write nothing."""
+    cols = 8 * pieces
+    g = torch.Generator(device=device).manual_seed(pieces)
+    buf = torch.full((3, cols + 8), 1e4, device=device, dtype=torch.bfloat16)
+    x = buf[:, :cols]
+    x.copy_(torch.randn(3, cols, generator=g, device=device))
+    w = (1 + 0.1 * torch.randn(cols, generator=g, device=device)).to(torch.bfloat16)
+    r = torch.randn(3, cols, generator=g, device=device).to(torch.bfloat16) if with_residual else None
+    _close_within_one_ulp(fused_rmsnorm(x, w, r), _eager_rmsnorm(x, w, r, 1e-6), f"rmsnorm {pieces} pieces")
+
+
 def test_strided_rows(device):
     """Row views of wider buffers (a fused gate/up projection's halves)."""
     g = torch.Generator(device=device).manual_seed(3)
