@@ -27,6 +27,8 @@
 //                   lane with v_perm_b32, because MFMA row m of product i stands
 //                   for d = 8*m + i. P^T comes straight out of the S^T
 //                   accumulator layout. No LDS is used.
+#include <type_traits>
+
 #include "attention_common.h"
 #include "prefill_tile.h"
 
@@ -1098,38 +1100,48 @@ __device__ __forceinline__ void decode_merge_body(const AttnParams& p, const int
       const int slot = i == 0 ? slot0 : 0;
       return (((int64_t)(wr * p.n_hgroups + hg) * 2 + slot) * p.hpw + wave) * p.rmax + r;
     };
-    // pieces four at a time: every load of a batch is issued before any is used (one
-    // memory round trip per batch), then merged into the running (max, sum, output)
+    // pieces in batches: every load of a batch is issued before any is used (one memory
+    // round trip per batch), then merged into the running (max, sum, output). A sequence of
+    // a small batch is cut into many pieces (23 of 179 keys for 4096 tokens of 37
+    // sequences), so beyond four they go eight at a time (with a thread for every output,
+    // that call 42.2 -> 41.0 us; 256 sequences to 8192 tokens, few pieces each, 246.4 both).
     float mmax = kNegBig, lsum = 0.f;
     f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
-    for (int i0 = 0; i0 < np; i0 += 4) {
-      float mv[4], lv[4];
-      f32x4 a0[4], a1[4];
+    auto merge = [&](auto batch) __attribute__((always_inline)) {
+      constexpr int N = batch;
+      for (int i0 = 0; i0 < np; i0 += N) {
+        float mv[N], lv[N];
+        f32x4 a0[N], a1[N];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t pi = piece(min(i0 + j, np - 1));
-        mv[j] = p.ws_ml[pi * 2];
-        lv[j] = p.ws_ml[pi * 2 + 1];
-        const f32x4* po = reinterpret_cast<const f32x4*>(p.ws_o + pi * D + 8 * c);
-        a0[j] = po[0];
-        a1[j] = po[1];
+        for (int j = 0; j < N; ++j) {
+          const int64_t pi = piece(min(i0 + j, np - 1));
+          mv[j] = p.ws_ml[pi * 2];
+          lv[j] = p.ws_ml[pi * 2 + 1];
+          const f32x4* po = reinterpret_cast<const f32x4*>(p.ws_o + pi * D + 8 * c);
+          a0[j] = po[0];
+          a1[j] = po[1];
+        }
+        float mx = mmax;
+#pragma unroll
+        for (int j = 0; j < N; ++j) mx = i0 + j < np ? fmaxf(mx, mv[j]) : mx;
+        const float keep = fast_exp2(mmax - mx);
+        lsum *= keep;
+        o0 *= keep;
+        o1 *= keep;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const float f = i0 + j < np ? fast_exp2(mv[j] - mx) : 0.f;
+          lsum += lv[j] * f;
+          o0 += a0[j] * f;
+          o1 += a1[j] * f;
+        }
+        mmax = mx;
       }
-      float mx = mmax;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) mx = i0 + j < np ? fmaxf(mx, mv[j]) : mx;
-      const float keep = fast_exp2(mmax - mx);
-      lsum *= keep;
-      o0 *= keep;
-      o1 *= keep;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float f = i0 + j < np ? fast_exp2(mv[j] - mx) : 0.f;
-        lsum += lv[j] * f;
-        o0 += a0[j] * f;
-        o1 += a1[j] * f;
-      }
-      mmax = mx;
-    }
+    };
+    if (np <= 4)
+      merge(std::integral_constant<int, 4>{});
+    else
+      merge(std::integral_constant<int, 8>{});
     const int j = r / p.n_rep;
     const int hq = (hg * p.hpw + wave) * p.n_rep + (r - j * p.n_rep);
     if constexpr (D <= 128) {
@@ -1305,9 +1317,9 @@ static int launch_decode_typed(AttnParams p, int max_query_len, char* ws, int64_
     defer->n_wg = n_wg;
     return SS_OK;
   }
-  // a shared-prefix merge folds S prefix parts into each of its rows' 8-d pieces (28 x
-  // 16 per C4 sequence): 512 threads give every piece its own thread
-  const int merge_threads = p.px_n > 0 ? 512 : 256;
+  // a thread merges 8 columns of a row, one after another if there are more than threads:
+  // 512 where a workgroup's heads have more than 256 (28 rows of 128 columns: 448)
+  const int merge_threads = p.px_n > 0 || p.hpw * p.n_rep * (D / 8) > 256 ? 512 : 256;
   hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3(n_wg + p.batch), dim3(merge_threads), 0, stream, p, n_wg, 0);
   return ss_host::launch_status("paged attention decode merge");
 }

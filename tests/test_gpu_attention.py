@@ -198,6 +198,22 @@ def test_decode_ignores_stale_nan_slots(device, lens):
     assert_attn_close(out, ref, f"stale NaN lens={lens}")
 
 
+@pytest.mark.parametrize("heads,dtype,tq", [((28, 4, 128), torch.bfloat16, 1), ((14, 2, 64), torch.float16, 1),
+                                            ((32, 8, 128), torch.bfloat16, 2)])
+@pytest.mark.parametrize("lens", [[4001], [5000, 37, 2500], [1100 + 130 * i for i in range(30)]])
+def test_decode_many_pieces_per_sequence(device, heads, dtype, tq, lens):
+    """Sequences cut into one to over a hundred pieces by the ranges, either side of a batch
+    of four and of multiples of eight; heads with fewer and more outputs than a merge
+    workgroup has threads."""
+    n_q, n_kv, d = heads
+    b = workloads.build_batch(lens, [tq] * len(lens), n_q=n_q, n_kv=n_kv, head_dim=d, block_size=16, dtype=dtype,
+                              device="cpu", seed=len(lens) + tq)
+    ref = _oracle_padded(b)
+    _to(b, device)
+    out = paged_attention_decode(b.padded_q(), b.kv_cache, b.block_tables, b.context_lens, 0, b.scale, b.block_size)
+    assert_attn_close(out, ref, f"decode pieces {heads} tq={tq} of {len(lens)}")
+
+
 def test_decode_head_dim_64_and_256(device):
     for d in (64, 256):
         b = workloads.build_batch([5, 77, 600], [1, 1, 1], n_q=16, n_kv=4, head_dim=d, block_size=16,
