@@ -30,7 +30,7 @@
 // partials in range order. Batch 1 takes a bandwidth GEMV. In every case the
 // result does not depend on timing.
 //
-// Group kernel (w4a16_group.hip): m <= 32 with groups of 32 or 64 keys, or a number of
+// Group kernel (w4a16_group.hip): m <= 64 with groups of 32 or 64 keys, or a number of
 // stages the skinny and tiled kernels do not split. Panel kernel (w4a16_panel.hip): m > 64
 // where the matrix cores set the time.
 //
@@ -1570,7 +1570,7 @@ struct W4Plan {
   int st;       // skinny: 128-key stages per wave
   bool panel;   // the panel kernel (m > 64, the matrix cores' shapes)
   PanelPlan pp;
-  bool group;   // the group kernel (m <= 64, groups of 32 or 64, or stages the others cannot split)
+  bool group;   // the group kernel (m <= 64 with groups of 32 or 64, or stages the others cannot split; scale tables past the LDS)
   GroupPlan gp;
   int mt, ns, kw, pf;
   int m_blocks, n_tiles;
@@ -1849,11 +1849,13 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
   const size_t red = (size_t)(pl.kw - 1) * pl.mt * pl.ns * 64 * 16;
   const size_t szb = (size_t)16 * pl.ns * (2 * groups + 2) * 4;
   pl.lds = szb > red ? szb : red;  // the reduction reuses the table's bytes
-  // the group kernel up to 32 rows, above them for N <= 4096 (m = 64, g = 64: 4864 x 896
-  // 24.6 against 35.5 us, 14336 x 4096 70 against 93; m = 40, 4096 x 6144 32 against 28),
-  // and where the scale table does not fit (m = 16, g = 32, 14336 x 4096 on the scalar
-  // kernel 1460 us, here 27)
-  if ((m <= 32 || n <= 4096 || pl.lds > kLdsBudget) && plan_w4a16_group(pl.gp, m, n, k, g)) {
+  // the group kernel up to 32 rows, up to 64 for N <= 4096 (m = 64, g = 64: 4864 x 896
+  // 24.6 against 35.5 us, 14336 x 4096 70 against 93; m = 40, 4096 x 6144 32 against 28;
+  // above 64 rows it reads and unpacks the weights again for every 64, and twice the
+  // untiled kernel's activations: 2176 x 4096 at m = 256 46 against 24 us, 7296 x 4096 at
+  // m = 2240 1066 against 584), and where the scale table does not fit (m = 16, g = 32,
+  // 14336 x 4096 on the scalar kernel 1460 us, here 27)
+  if ((m <= 32 || (m <= 64 && n <= 4096) || pl.lds > kLdsBudget) && plan_w4a16_group(pl.gp, m, n, k, g)) {
     pl.group = true;
     pl.m_blocks = pl.gp.m_blocks;
   }

@@ -1,5 +1,6 @@
 // W4A16 group kernel (m <= 64, groups of 32, 64 or 128 keys, any whole number of 128-key
-// stages): small products, where the time is a few memory round trips.
+// stages): small products, where the time is a few memory round trips. (Above 64 rows it
+// runs only where the untiled kernel's scale table does not fit its LDS.)
 //
 // A workgroup owns 16 NS weight rows and 16 MT activation rows; its waves (up to sixteen)
 // split K into contiguous runs of 128-key stages, and each wave requests the weights,

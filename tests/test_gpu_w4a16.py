@@ -268,6 +268,18 @@ def test_group_kernel(device, m, k, n, g, act, sdt):
     assert torch.equal(w4a16_gemm(xs, qd, sd, zd, g), y)
 
 
+@pytest.mark.parametrize("m,k,g", [(65, 2176, 128), (512, 896, 128), (300, 1152, 64), (130, 640, 32)])
+def test_rows_past_64_keep_the_untiled_kernel(device, m, k, g):
+    """Above 64 rows, linears that the tiled kernels do not split run on the untiled kernel
+    on both sides of N = 4096: a weight row's results are the same bits whether the call has
+    4096 rows or 4112 (the group kernel adds K in another order, and is slower here)."""
+    x, qw, s, z, ref = _host_case(4112, k, m, g, seed=m + k, act=torch.bfloat16, sdt=torch.float16, zeros="random")
+    xd, qd, sd, zd = x.to(device), qw.to(device), s.to(device), z.to(device)
+    y = w4a16_gemm(xd, qd, sd, zd, g)
+    _assert_close(y, ref, f"untiled m={m} k={k} g={g}")
+    assert torch.equal(w4a16_gemm(xd, qd[:4096], sd[:4096], zd[:4096], g), y[:, :4096])
+
+
 # (plans as the host computes them for 256 CUs: panels of 16 MT rows, 256- or 128-row weight tiles)
 @pytest.mark.parametrize("m,k,n,act,sdt", [
     # four weight tiles a wave
