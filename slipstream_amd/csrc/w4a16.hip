@@ -16,7 +16,7 @@
 // (k0,k4),(k1,k5),(k2,k6),(k3,k7) of each word, and every activation fragment is
 // permuted the same way in registers (v_perm_b32), so the dot products pair up.
 //
-// Untiled kernel (w4a16_kernel, m > 32 where the tiled kernels do not take the shape): a workgroup owns 16*NS weight rows and 16*MT
+// Untiled kernel (w4a16_kernel): a workgroup owns 16*NS weight rows and 16*MT
 // activation rows; its KW waves split K into contiguous slices (each wave streams
 // its own slice of the rows: coalesced 16-byte loads, the next block in flight
 // while the current one computes), and one LDS pass adds the slices in wave
@@ -48,14 +48,18 @@ namespace {
 // MT: 16-row activation tiles; NS: 16-row weight tiles; BIT: 128-key iterations
 // per pipeline block; WIDE: g % 128 == 0 (one group per iteration, a lane holds 32
 // consecutive keys of its row: one 16-byte load), else g % 32 == 0 (one group per
-// 32-key MFMA step, 4-byte loads). Every wave loads its own activation fragments and sums
-// them with an all-ones MFMA.
+// 32-key MFMA step, 4-byte loads); XLDS: the workgroup's activation rows (all of K,
+// permuted) and their per-fold sums are staged in LDS once -- used when they fit;
+// otherwise every wave loads its own activation fragments and sums them with an
+// all-ones MFMA.
 //
-// Dynamic LDS: the scale table, 16*NS rows x (2*groups + 2) floats, pairs (s, s*(MAGIC+z)),
+// Dynamic LDS: [XLDS: x rows (K + 8 elements each) | fold sums [K/UNIT][16*MT]]
+//              [scale table: 16*NS rows x (2*groups + 2) floats, pairs (s, s*(MAGIC+z))]
 // and, once every wave is past the main loop, the same bytes again as the
 // reduction buffer (kw - 1) x MT*NS x 64 x f32x4.
-template <typename T, int MT, int NS, int BIT, bool WIDE>
+template <typename T, int MT, int NS, int BIT, bool WIDE, bool XLDS>
 __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
+  constexpr int UNIT = WIDE ? 128 : 32;  // keys per fold (one quantisation group; 4 per 128-key iteration if !WIDE)
   typedef W4Elem<T> E;
   extern __shared__ __attribute__((aligned(16))) char s_dyn[];
 
@@ -71,10 +75,14 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
   const int per = (iters + p.kw - 1) / p.kw;
   const int it0 = wave * per;
   const int it1 = min(iters, it0 + per);
+  const int lrow = p.k + 8;           // LDS row of x, elements (16-byte skew per row)
   const int szrow = 2 * p.groups + 2;  // LDS row of the scale table, floats (8-byte skew per row)
   const uint32_t magic = in_vgpr(E::kMagicPair);
 
-  float* s_sz = (float*)s_dyn;
+  T* s_x = (T*)s_dyn;
+  const size_t x_bytes = XLDS ? (size_t)rows * lrow * sizeof(T) + (size_t)(p.k / UNIT) * 16 * MT * 4 : 0;
+  float* s_xs = (float*)(s_dyn + (XLDS ? (size_t)rows * lrow * sizeof(T) : 0));
+  float* s_sz = (float*)(s_dyn + x_bytes);
   f32x4* s_red = (f32x4*)s_dyn;  // aliases the tables above, used after a barrier
 
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(p.qw, (uint32_t)((int64_t)p.n * p.k / 2));
@@ -89,7 +97,7 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
     u32x4 w[NS][BIT];
   };
   struct XBlock {
-    u32x4 x[MT][BIT][4];
+    u32x4 x[XLDS ? 1 : MT][XLDS ? 1 : BIT][4];
   };
 
   // Weight loads only (no use), always in range: iterations past the slice reload
@@ -147,6 +155,25 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
       }
     }
   }
+  if (XLDS) {
+    // rows [m0, m0 + rows) of x for all of K, permuted, plus their fold sums
+    constexpr int GL = UNIT / 8;  // staging lanes per fold (consecutive lanes)
+    const int cols = p.k / 8;
+    for (int q = threadIdx.x; q < rows * cols; q += blockDim.x) {
+      const int r = q / cols, c = q - r * cols;
+      const u32x4 v = load16((const T*)p.x + (int64_t)(m0 + r) * p.x_stride + 8 * c);
+      store16(&s_x[r * lrow + 8 * c], permute_x(v));
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum += E::to_f32(v[j] & 0xFFFFu) + E::to_f32(v[j] >> 16);
+#pragma unroll
+      for (int o = 1; o < GL; o <<= 1) sum += __shfl_xor(sum, o);
+      if (c % GL == 0) s_xs[(c / GL) * 16 * MT + r] = sum;
+    }
+    // sums of rows past M are 0 (their outputs are never stored)
+    for (int q = threadIdx.x; q < (p.k / UNIT) * 16 * MT; q += blockDim.x)
+      if (q % (16 * MT) >= rows) s_xs[q] = 0.f;
+  }
   __syncthreads();
 
   // Activation rows past M read row M-1 (a valid address); they only feed output
@@ -159,9 +186,11 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
   const __amdgpu_buffer_rsrc_t rx = buffer_rsrc(
       (const T*)p.x + (int64_t)m0 * p.x_stride, (uint32_t)(((int64_t)(rows - 1) * p.x_stride + p.k) * sizeof(T)));
   int xrow[MT];  // byte offset of this lane's activation row
+  int xl[MT];    // LDS row (XLDS)
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     xrow[mt] = (int)((int64_t)min(mt * 16 + ln, rows - 1) * p.x_stride * (int64_t)sizeof(T));
+    xl[mt] = min(mt * 16 + ln, rows - 1) * lrow;
   }
 
   f32x4 acc[MT][NS];
@@ -171,6 +200,7 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
     for (int ns = 0; ns < NS; ++ns) acc[mt][ns] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   auto load_x = [&](int itb, XBlock& xb) {
+    if (XLDS) return;
 #pragma unroll
     for (int it = 0; it < BIT; ++it) {
       // the iteration's key offset is uniform: it rides in the scalar offset, so the
@@ -182,7 +212,7 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
         const int klane = (WIDE ? 32 * kg + 8 * s : 32 * s + 8 * kg) * (int)sizeof(T);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
-          xb.x[mt][it][s] = __builtin_bit_cast(
+          xb.x[XLDS ? 0 : mt][XLDS ? 0 : it][s] = __builtin_bit_cast(
               u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xrow[mt] + klane, kk, 0));
       }
     }
@@ -208,8 +238,12 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
         u32x4 a[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          a[mt] = permute_x(xb.x[mt][it][s]);
-          X[mt] = Elem<T>::mfma(a[mt], ones, X[mt]);
+          if (XLDS) {
+            a[mt] = load16(&s_x[xl[mt] + kk + (WIDE ? 32 * kg + 8 * s : 32 * s + 8 * kg)]);
+          } else {
+            a[mt] = permute_x(xb.x[XLDS ? 0 : mt][XLDS ? 0 : it][s]);
+            X[mt] = Elem<T>::mfma(a[mt], ones, X[mt]);
+          }
         }
 #pragma unroll
         for (int ns = 0; ns < NS; ++ns) {
@@ -219,6 +253,11 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
         }
         if (!WIDE || s == 3) {  // end of a fold unit: fold it into acc
           const int kf = kk + (WIDE ? 0 : 32 * s);
+          if (XLDS) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+              X[mt] = *reinterpret_cast<const f32x4*>(&s_xs[(kf / UNIT) * 16 * MT + mt * 16 + 4 * kg]);
+          }
           const int gi = kf / p.g;
 #pragma unroll
           for (int ns = 0; ns < NS; ++ns) {
@@ -1562,6 +1601,7 @@ __global__ __launch_bounds__(512) void w4a16_narrow_kernel(const W4Params p) {
 struct W4Plan {
   bool fast;
   bool wide;
+  bool xlds;   // untiled kernel: activations staged in LDS
   int narrow;  // activation rows of the narrow kernel (1, 2 or 4), 0: not used
   int gemv;  // 1: the batch-1 GEMV kernel
   bool tile;  // the tiled kernel (activations shared through LDS)
@@ -1788,6 +1828,33 @@ bool plan_wide(W4Plan& pl, int64_t m, int64_t n, int64_t k, int g) {
 
 constexpr size_t kLdsBudget = 64 * 1024;  // LDS bytes per workgroup
 
+// The group kernel against the untiled one (pl holds the latter's form), both measured over
+// one to 64 rows, 1 to 119 stages and N from 128 to 32768, weights from HBM.
+// Groups of 32 or 64 keys: up to 32 rows, and up to 64 for N <= 4096 (m = 64, g = 64: 4864 x
+// 896 24.6 against 35.5 us, 14336 x 4096 70 against 93; m = 40, 4096 x 6144 32 against 28).
+// Above 64 rows it reads and unpacks the weights again for every 64, and twice the untiled
+// kernel's activations: 2176 x 4096 at m = 256 46 against 24 us, 7296 x 4096 at m = 2240
+// 1066 against 584.
+// Groups of whole stages (shapes that the skinny and tiled kernels do not split): up to
+// 4096 weight rows, one workgroup of 16 per CU (7296 x 4096 at m = 17 14.4 against 18.9 us,
+// 896 to 8064 x 4096 1.04 to 1.5 times as fast), except one or two rows of more than 64
+// stages in fewer workgroups than CUs, where each wave makes a second round trip (9344 x
+// 1536 at m = 1 0.88 times). With more weight rows a CU takes several workgroups and the
+// round trips of a long K add up in each, while the untiled kernel prefetches: 4864 x 6144
+// at m = 32 0.72 to 0.75 times from 39 stages, 7296 x 9728 at m = 1 22 against 16 us. So
+// only short K: from 4 stages (below, the launch is all there is: 1 stage 0.8 to 0.95
+// times) to 23 (2944 x 8192 at m = 16 1.6 times, m = 24 1.2), to 16 where a tile of up to 16 rows
+// has more than two workgroups a CU (2432 x 16400 at m = 1 0.85), to 12 where two tiles of
+// rows have fewer (1920 x 6144 at m = 32 0.88).
+bool group_kernel_wins(const W4Plan& pl, int64_t m, int64_t n, int64_t k) {
+  const int64_t stages = k / 128, round = 16LL * ss_host::device_cu_count();  // weight rows of one workgroup per CU
+  if (m > 64 || (m > 32 && n > 4096)) return false;
+  if (!pl.wide) return true;
+  if (n <= round) return !(pl.xlds && m <= 2 && stages > 64 && n + 15 < round);
+  const int64_t most = m <= 16 ? (n <= 2 * round ? 23 : 16) : (n < 2 * round ? 12 : 23);
+  return stages >= 4 && stages <= most;
+}
+
 W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow_tile = true, bool allow_panel = true) {
   W4Plan pl = {};
   pl.fast = act16 && k % 128 == 0 && g % 32 == 0 && k > 0 && n * k / 2 < ((int64_t)1 << 31);
@@ -1838,8 +1905,25 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
   pl.tile = false;
   const int64_t groups = k / g;
   const int iters = (int)(k / 128);
-  const int64_t want = 8LL * ss_host::device_cu_count();  // waves in flight to cover HBM latency
-  pl.mt = 4, pl.ns = 2;
+  const int64_t cus = ss_host::device_cu_count();
+  const int64_t want = 8LL * cus;  // waves in flight to cover HBM latency
+  // the untiled kernel's form. Groups of whole stages: x staged in LDS when one 16-row tile
+  // of it fits beside the scale table; other groups reach it above 32 rows only
+  const int64_t rows1 = m < 16 ? m : 16;
+  const size_t x1 = (size_t)rows1 * (k + 8) * 2 + (size_t)(k / 128) * 16 * 4;
+  const size_t sz1 = (size_t)16 * (2 * groups + 2) * 4;
+  if (pl.wide && m <= 16 && x1 + sz1 <= kLdsBudget) {
+    pl.mt = 1, pl.ns = 1, pl.xlds = true;
+  } else if (pl.wide && m <= 16) {
+    // 64 weight rows share each activation fragment, unless that leaves more than
+    // half the CUs idle: then 32 (twice the activation reads, twice the workgroups;
+    // measured faster for N = 4096 and 6144, slower for 14336)
+    pl.mt = 1, pl.ns = (n + 63) / 64 >= cus / 2 ? 4 : 2;
+  } else if (pl.wide && m <= 32) {
+    pl.mt = 2, pl.ns = 2;
+  } else {
+    pl.mt = 4, pl.ns = 2;
+  }
   pl.m_blocks = (int)((m + 16 * pl.mt - 1) / (16 * pl.mt));
   pl.n_tiles = (int)((n + 16 * pl.ns - 1) / (16 * pl.ns));
   // K slices per workgroup, with at least two 128-key iterations per slice
@@ -1847,15 +1931,12 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
   pl.kw = wgs * 4 >= want ? 4 : kMaxKW;
   while (pl.kw > 1 && iters < 2 * pl.kw) pl.kw >>= 1;
   const size_t red = (size_t)(pl.kw - 1) * pl.mt * pl.ns * 64 * 16;
+  const size_t xb = pl.xlds ? x1 : 0;
   const size_t szb = (size_t)16 * pl.ns * (2 * groups + 2) * 4;
-  pl.lds = szb > red ? szb : red;  // the reduction reuses the table's bytes
-  // the group kernel up to 32 rows, up to 64 for N <= 4096 (m = 64, g = 64: 4864 x 896
-  // 24.6 against 35.5 us, 14336 x 4096 70 against 93; m = 40, 4096 x 6144 32 against 28;
-  // above 64 rows it reads and unpacks the weights again for every 64, and twice the
-  // untiled kernel's activations: 2176 x 4096 at m = 256 46 against 24 us, 7296 x 4096 at
-  // m = 2240 1066 against 584), and where the scale table does not fit (m = 16, g = 32,
-  // 14336 x 4096 on the scalar kernel 1460 us, here 27)
-  if ((m <= 32 || (m <= 64 && n <= 4096) || pl.lds > kLdsBudget) && plan_w4a16_group(pl.gp, m, n, k, g)) {
+  pl.lds = xb + szb > red ? xb + szb : red;  // the reduction reuses the tables' bytes
+  // The group kernel where it is the faster one (group_kernel_wins), and where the scale
+  // table does not fit (m = 16, g = 32, 14336 x 4096 on the scalar kernel 1460 us, here 27).
+  if ((group_kernel_wins(pl, m, n, k) || pl.lds > kLdsBudget) && plan_w4a16_group(pl.gp, m, n, k, g)) {
     pl.group = true;
     pl.m_blocks = pl.gp.m_blocks;
   }
@@ -1863,15 +1944,21 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
   return pl;
 }
 
+template <typename T, int MT, int NS, int BIT, bool WIDE, bool XLDS>
+int launch_w4a16_form(const W4Params& p, const W4Plan& pl, hipStream_t stream) {
+  dim3 grid((unsigned)pl.n_tiles, (unsigned)pl.m_blocks);
+  hipLaunchKernelGGL((w4a16_kernel<T, MT, NS, BIT, WIDE, XLDS>), grid, dim3(64 * pl.kw), pl.lds, stream, p);
+  return ss_host::launch_status("w4a16 gemm");
+}
+
 template <typename T>
 int launch_w4a16_untiled(const W4Params& p, const W4Plan& pl, hipStream_t stream) {
-  dim3 grid((unsigned)pl.n_tiles, (unsigned)pl.m_blocks);
-  dim3 block(64 * pl.kw);
-  if (pl.wide)
-    hipLaunchKernelGGL((w4a16_kernel<T, 4, 2, 1, true>), grid, block, pl.lds, stream, p);
-  else
-    hipLaunchKernelGGL((w4a16_kernel<T, 4, 2, 1, false>), grid, block, pl.lds, stream, p);
-  return ss_host::launch_status("w4a16 gemm");
+  if (!pl.wide) return launch_w4a16_form<T, 4, 2, 1, false, false>(p, pl, stream);
+  if (pl.xlds) return launch_w4a16_form<T, 1, 1, 4, true, true>(p, pl, stream);
+  if (pl.mt == 1 && pl.ns == 4) return launch_w4a16_form<T, 1, 4, 2, true, false>(p, pl, stream);
+  if (pl.mt == 1) return launch_w4a16_form<T, 1, 2, 2, true, false>(p, pl, stream);
+  if (pl.mt == 2) return launch_w4a16_form<T, 2, 2, 2, true, false>(p, pl, stream);
+  return launch_w4a16_form<T, 4, 2, 1, true, false>(p, pl, stream);
 }
 
 // Tag of a split call's arrival words: a process-wide count, so that words left by earlier

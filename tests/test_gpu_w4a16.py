@@ -280,6 +280,32 @@ def test_rows_past_64_keep_the_untiled_kernel(device, m, k, g):
     assert torch.equal(w4a16_gemm(xd, qd[:4096], sd[:4096], zd[:4096], g), y[:, :4096])
 
 
+# (untiled forms as the host computes them for 256 CUs)
+@pytest.mark.parametrize("m,k,n,act,sdt,staged", [
+    (1, 7296, 8240, torch.bfloat16, torch.float16, True),    # one row in LDS
+    (2, 8832, 1000, torch.float16, torch.bfloat16, True),    # more than 64 stages, fewer workgroups than CUs
+    (1, 256, 8200, torch.bfloat16, torch.float32, True),     # two stages
+    (5, 5888, 4100, torch.float16, torch.float16, True),
+    (16, 7296, 9728, torch.bfloat16, torch.float16, False),  # four weight tiles
+    (12, 4992, 4356, torch.float16, torch.bfloat16, False),  # two weight tiles
+    (32, 1664, 4200, torch.bfloat16, torch.float32, False),  # two activation tiles, 13 stages
+    (17, 7296, 4356, torch.bfloat16, torch.float16, False),  # two activation tiles, the second of one row
+])
+def test_whole_stage_groups_on_the_untiled_kernel(device, m, k, n, act, sdt, staged):
+    """Groups of 128 keys where the group kernel's repeated round trips lose (a CU has several
+    of its workgroups, and K is long) run on the untiled kernel's forms for up to 32 rows.
+    Against the oracle; where the activations are not staged in LDS, whose sums are added in
+    another order, a row has the same bits as in a call of 33 rows, which only the untiled
+    kernel takes."""
+    x, qw, s, z, ref = _host_case(n, k, 33, 128, seed=m + k + n, act=act, sdt=sdt, zeros="random")
+    xd, qd, sd, zd = x.to(device), qw.to(device), s.to(device), z.to(device)
+    y = w4a16_gemm(xd[:m], qd, sd, zd, 128)
+    _assert_close(y, ref[:m], f"untiled m={m} k={k} n={n}")
+    assert torch.equal(y, w4a16_gemm(xd[:m], qd, sd, zd, 128))
+    if not staged:
+        assert torch.equal(y, w4a16_gemm(xd, qd, sd, zd, 128)[:m])
+
+
 # (plans as the host computes them for 256 CUs: panels of 16 MT rows, 256- or 128-row weight tiles)
 @pytest.mark.parametrize("m,k,n,act,sdt", [
     # four weight tiles a wave
