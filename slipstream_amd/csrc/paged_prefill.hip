@@ -256,7 +256,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // A prefill with fewer items than CUs (a chunk alone: 256 tokens of a 32/8-head model are 64
 // items) leaves most of the chip idle and its few workgroups walk the keys alone: the keys
 // of every item are split over workgroups (prefill_split_kernel), fp32 partial rows and
-// their (max, sum) go to the workspace, and prefill_split_merge_kernel adds them.
+// their (max, sum) go to the workspace, and prefill_split_merge_kernel adds them. How many
+// parts an item has is decided on the device, from its sequence's length: the host knows
+// only the table's width, which an engine pads to its longest sequence.
 template <typename T, int D>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_split_kernel(
     const AttnParams p) {
@@ -270,28 +272,35 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(const AttnPara
   constexpr int TPR = D / 4;  // threads of a row
   const int64_t r = ((int64_t)blockIdx.x * 256 + threadIdx.x) / TPR;
   const int d = 4 * (threadIdx.x % TPR);
-  const int item = (int)(r >> 7), row = (int)(r & 127);
+  constexpr int BLOCKS = 128 * TPR / 256;  // of an item
+  const int item = blockIdx.x / BLOCKS, row = (int)(r & 127);
   const int entry = item / p.n_kv, h = item - entry * p.n_kv;
   const int b = entry / p.work_qtiles, qt = p.work_qtiles - 1 - (entry - b * p.work_qtiles);
-  const int rr = qt * 128 + row;
-  if (b >= p.batch || rr >= p.tq * p.n_rep) return;
+  const int rr = qt * 128 + row, R = p.tq * p.n_rep;
+  // the item's parts, as prefill_tile_body has them; one part is written already
+  const int ctx = kv_len(p, b), kvt = seq_kv_tokens(p, ctx);
+  const int kv_all = min(kvt, ctx - p.tq + min(R - 1, qt * 128 + 127) / p.n_rep + 1);
+  const int tiles_all = kv_all > 0 ? (kv_all + 63) / 64 : 0;
+  const int per_part = split_part_tiles(p.split, tiles_all, (kvt + 63) / 64);
+  if (tiles_all <= per_part || rr >= R) return;
+  const int parts = (tiles_all + per_part - 1) / per_part;
   const int64_t base = ((int64_t)item * p.split) * 128 + row;
   float mx = kNegBig;
-  for (int i = 0; i < p.split; ++i) mx = fmaxf(mx, p.ws_ml[2 * (base + 128 * i)]);
+  for (int i = 0; i < parts; ++i) mx = fmaxf(mx, p.ws_ml[2 * (base + 128 * i)]);
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
   float l = 0.f;
-  for (int i0 = 0; i0 < p.split; i0 += 4) {
+  for (int i0 = 0; i0 < parts; i0 += 4) {
     f32x4 x[4];
     float2 ml[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int64_t at = base + 128 * min(i0 + i, p.split - 1);
+      const int64_t at = base + 128 * min(i0 + i, parts - 1);
       ml[i] = *reinterpret_cast<const float2*>(p.ws_ml + 2 * at);
       x[i] = *reinterpret_cast<const f32x4*>(p.ws_o + at * D + d);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float w = i0 + i < p.split && ml[i].y > 0.f ? fast_exp2(ml[i].x - mx) : 0.f;
+      const float w = i0 + i < parts && ml[i].y > 0.f ? fast_exp2(ml[i].x - mx) : 0.f;
       l = fmaf(w, ml[i].y, l);
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = fmaf(w, x[i][e], o[e]);
@@ -303,17 +312,17 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(const AttnPara
   *reinterpret_cast<u32x2*>(out) = u32x2{Elem<T>::pack2(o[0] * inv, o[1] * inv), Elem<T>::pack2(o[2] * inv, o[3] * inv)};
 }
 
-// Key parts per item of a padded prefill: as many as keep one workgroup per CU, of at least
-// three 64-key tiles of the widest table, within the workspace; 1: not split. Where two
+// Most key parts of an item of a padded prefill: as many as keep one workgroup per CU, of at
+// least kPartTiles of the widest table, within the workspace; 1: not split. Where two
 // parts just fit it still pays (512 tokens over 2000, 128 items: 58.5 -> 42.4 us).
 int prefill_split(const AttnParams& p, int64_t items, int head_dim, int64_t ws_bytes) {
   const int64_t tiles = (((int64_t)p.max_blocks << p.bs_shift) + 63) / 64;
   int64_t s = ss_host::device_cu_count() / items;
-  s = s < tiles / 3 ? s : tiles / 3;
+  s = s < tiles / kPartTiles ? s : tiles / kPartTiles;
   s = s < 16 ? s : 16;
   const int64_t part = items * 128 * (head_dim + 2) * 4;
   while (s > 1 && s * part > ws_bytes) --s;
-  return s < 1 ? 1 : (int)s;
+  return s < 2 || tiles < split_least_tiles((int)s) ? 1 : (int)s;
 }
 
 // The tiled prefill's work list (plan_work_list) built by a one-workgroup launch, when

@@ -109,6 +109,18 @@ __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
+// Tiles of a key part of an item of tiles_all tiles whose sequence's last row has seq_tiles.
+// The partial rows and their merge cost what five to seven tiles of the walk do, and two parts
+// save only half of it: a sequence of fewer than 8 + 12 / split tiles is walked whole, and a
+// part has at least kPartTiles (32/8 heads of 128, whole against split: 256 tokens over 460,
+// twice, two parts of 12 tiles 25.1 against 27.8 us, over 600, 14 tiles, 28.0 both; 256 over 460 once,
+// four parts 24.2 against 23.0; 64 over 460 once, nine tiles in three parts 19.7 against 16.8).
+constexpr int kPartTiles = 3;
+__device__ __host__ __forceinline__ int split_least_tiles(int split) { return 8 + 12 / split; }
+__device__ __forceinline__ int split_part_tiles(int split, int tiles_all, int seq_tiles) {
+  return seq_tiles < split_least_tiles(split) ? max(tiles_all, 1) : max(kPartTiles, (seq_tiles + split - 1) / split);
+}
+
 extern __shared__ __attribute__((aligned(1024))) char s_tile_stages[];
 
 // Work split: a workgroup covers 128 query rows of one (sequence, KV head) with
@@ -123,9 +135,10 @@ extern __shared__ __attribute__((aligned(1024))) char s_tile_stages[];
 // for the occupancy that size alone allows.
 // The body of prefill_tile_kernel as workgroup wg of G (the shared-prefix cascade runs
 // it in the first G workgroups of a launch whose others run the decode).
-// SPLIT: the keys of every item in p.split contiguous parts of 64-key tiles, one workgroup
-// each (all entries in order, no list): fp32 partial rows into p.ws_o and their (max, sum)
-// into p.ws_ml, which prefill_split_merge_kernel combines.
+// SPLIT: the keys of an item in up to p.split contiguous parts of split_part_tiles 64-key
+// tiles, one workgroup each (all entries in order, no list; workgroups past an item's parts
+// have nothing to do): fp32 partial rows into p.ws_o and their (max, sum) into p.ws_ml, which
+// prefill_split_merge_kernel combines. An item of one part writes its output itself.
 template <typename T, int D, bool SPLIT = false>
 __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int* __restrict__ work, const int wg,
                                                   const int G) {
@@ -177,8 +190,10 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
   const int kv_all = p.noncausal ? kvt : min(kvt, ctx - qlen + last_row / p.n_rep + 1);
   const int tiles_all = kv_all > 0 ? (kv_all + C::KT - 1) / C::KT : 0;
   // this workgroup's tiles [t0, ntiles): all of them, or its part
-  const int per_part = SPLIT ? (tiles_all + p.split - 1) / p.split : tiles_all;
+  const int per_part = SPLIT ? split_part_tiles(p.split, tiles_all, (kvt + C::KT - 1) / C::KT) : tiles_all;
   const int t0 = SPLIT ? part * per_part : 0;
+  if (SPLIT && part > 0 && t0 >= tiles_all) return;
+  const bool partial = SPLIT && tiles_all > per_part;
   const int ntiles = SPLIT ? min(tiles_all, t0 + per_part) : tiles_all;
   const int kv_end = SPLIT ? min(kv_all, ntiles * C::KT) : kv_all;
   const ConstTable table = (ConstTable)(p.bt + (int64_t)b * p.bt_stride);
@@ -511,7 +526,7 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
   for (int nt = 0; nt < NT; ++nt) {
     const float lt = lsum[nt][0];
     const int rr = row0 + wave * 16 * NT + 16 * nt + n;
-    if constexpr (SPLIT) {
+    if (partial) {
       const int64_t prow = (int64_t)slot * ROWS + (rr - row0);
       if (g == 0) *reinterpret_cast<float2*>(p.ws_ml + 2 * prow) = float2{mrow[nt], lt};
       float* const o = p.ws_o + prow * D + (D / 4) * g;

@@ -445,6 +445,28 @@ def test_prefill_split_keys(device, heads, dtype, tq, ctx, width, bs):
     assert torch.equal(out, again)
 
 
+@pytest.mark.parametrize("heads,dtype,tq,ctx", [
+    ((32, 8, 128), torch.bfloat16, 64, [64]),
+    ((32, 8, 128), torch.bfloat16, 512, [512]),               # two parts would fit the CUs
+    ((28, 4, 128), torch.float16, 40, [40, 300, 560, 17]),    # nine tiles, the fewest split are ten; a row tile without a visible key
+    ((14, 2, 64), torch.float16, 131, [331, 500]),
+])
+def test_short_prefill_is_not_split(device, heads, dtype, tq, ctx):
+    """Sequences of a few key tiles are walked whole however wide their tables are (the
+    partial rows and their merge cost more than the walk): a padded call over tables of
+    8192 tokens gives the bits of the packed call, which never splits."""
+    n_q, n_kv, d = heads
+    b = workloads.build_batch(ctx, [tq] * len(ctx), n_q=n_q, n_kv=n_kv, head_dim=d, block_size=16, dtype=dtype,
+                              device=device, seed=tq + sum(ctx))
+    wide = torch.full((len(ctx), 512), -1, dtype=torch.int32, device=device)
+    wide[:, : b.block_tables.shape[1]] = b.block_tables
+    cu = torch.arange(len(ctx) + 1, dtype=torch.int32, device=device) * tq
+    want = paged_attention_varlen(b.q, b.kv_cache, wide, cu, b.context_lens, 0, b.scale, 16, tq)
+    for tables in (wide, b.block_tables):
+        out = paged_attention_prefill(b.padded_q(), b.kv_cache, tables, b.context_lens, 0, b.scale, 16)
+        assert torch.equal(out.reshape(want.shape), want)
+
+
 def test_prefill_head_dim_256(device):
     b = workloads.build_batch([40, 300], [40, 40], n_q=8, n_kv=2, head_dim=256, block_size=16,
                               dtype=torch.bfloat16, device="cpu", seed=256)
