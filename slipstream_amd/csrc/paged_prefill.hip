@@ -349,10 +349,20 @@ int launch_prefill_typed(const AttnParams& p, int max_query_len, int* work, int6
     constexpr int DD = D <= 128 ? D : 128;
     const int lds = 6 * TileCfg<T, DD>::PLANE;
     const int64_t items = (int64_t)p.batch * qtiles * p.n_kv;
+    const int64_t need = p.work_qtiles > 0 ? 0 : prefill_work_bytes(p.batch, p.n_rep, max_query_len);
+    if (p.work_qtiles > 0 && p.work_qtiles != qtiles) {
+      ss_host::set_error("paged attention prefill: %d implicit query tiles, the launch has %lld", p.work_qtiles,
+                         (long long)qtiles);
+      return SS_ERR_INVALID;
+    }
+    if (need > 0 && (!work || work_bytes < need)) {
+      ss_host::set_error("paged attention prefill: workspace of %lld bytes for the work list, needs %lld",
+                         (long long)work_bytes, (long long)need);
+      return SS_ERR_WORKSPACE;
+    }
     // (padded calls only: every sequence has the same query tiles, so all parts are written)
-    const int split = ws && ((uintptr_t)ws & 15) == 0 && !p.cu && !p.lse && p.chunk_tokens == 0 && p.work_qtiles == 0 && !planned && !p.noncausal
-                          ? prefill_split(p, items, DD, ws_bytes)
-                          : 1;
+    const bool padded = !p.cu && !p.lse && p.chunk_tokens == 0 && p.work_qtiles == 0 && !planned && !p.noncausal;
+    const int split = padded && ws && ((uintptr_t)ws & 15) == 0 ? prefill_split(p, items, DD, ws_bytes) : 1;
     if (split > 1) {
       static bool split_attr_set = false;  // per instantiation; the attribute is process-wide
       if (!split_attr_set) {
@@ -374,17 +384,6 @@ int launch_prefill_typed(const AttnParams& p, int max_query_len, int* work, int6
       hipLaunchKernelGGL((prefill_split_merge_kernel<T, DD>), dim3((unsigned)(items * 128 * (DD / 4) / 256)), dim3(256),
                          0, stream, ps);
       return ss_host::launch_status("paged attention prefill merge");
-    }
-    const int64_t need = p.work_qtiles > 0 ? 0 : prefill_work_bytes(p.batch, p.n_rep, max_query_len);
-    if (p.work_qtiles > 0 && p.work_qtiles != qtiles) {
-      ss_host::set_error("paged attention prefill: %d implicit query tiles, the launch has %lld", p.work_qtiles,
-                         (long long)qtiles);
-      return SS_ERR_INVALID;
-    }
-    if (need > 0 && (!work || work_bytes < need)) {
-      ss_host::set_error("paged attention prefill: workspace of %lld bytes for the work list, needs %lld",
-                         (long long)work_bytes, (long long)need);
-      return SS_ERR_WORKSPACE;
     }
     static bool attr_set = false;  // per instantiation; the attribute is process-wide
     if (!attr_set) {

@@ -174,6 +174,27 @@ def test_attention_workspace_holds_the_prefill_work_list():
     assert b"work list" in lib.ss_last_error()
 
 
+@pytest.mark.parametrize("batch,tq", [(4, 40), (1, 256)])
+def test_small_prefill_needs_the_work_lists_workspace(batch, tq):
+    """A small padded prefill over tables of 1024 tokens, whose keys would be split over
+    workgroups and which then uses no work list, is refused all the same with a workspace
+    that has no room for one: what fits does not depend on the kernels a call takes."""
+    from slipstream_amd import _ffi
+
+    lib = _ffi.lib()
+    need = ctypes.c_int64(0)
+    assert lib.ss_paged_attention_workspace_size(batch, 32, 8, 128, tq, _ffi.SS_DTYPE_BF16,
+                                                 ctypes.byref(need)) == _ffi.SS_OK
+    fake = 1 << 20  # 16-byte aligned, never dereferenced on the host
+    q_str = _ffi.i64_array([tq * 32 * 128, 128, 32 * 128])
+    o_str = _ffi.i64_array([tq * 32 * 128, 32 * 128, 128])
+    c_str = _ffi.i64_array([16 * 8 * 128, 8 * 128, 128])
+    st = lib.ss_paged_attention(fake, fake, fake, fake, fake, fake, batch, 32, 8, 128, tq, 64, 16, 1024,
+                                q_str, o_str, c_str, 64, 1.0, _ffi.SS_DTYPE_BF16, fake, need.value - 4, None)
+    assert st == _ffi.SS_ERR_WORKSPACE, lib.ss_last_error()
+    assert b"work list" in lib.ss_last_error()
+
+
 def test_shared_prefix_argument_errors_need_no_device():
     """The shared-prefix entry checks GQA, batch and prefix_blocks on the host; an empty
     batch returns SS_OK before any HIP call; the Python wrapper refuses CPU tensors."""
