@@ -55,7 +55,8 @@ struct AttnParams {
                       //   ctx_lens, and query tokens [b * q_period, (b + 1) * q_period)
   int work_qtiles;    // > 0: the prefill takes entry e = sequence e / work_qtiles, query tile
                       //   work_qtiles - 1 - e % work_qtiles, in order, instead of a work list
-  int split;          // prefill_split_kernel: key parts of an item (ws_o, ws_ml hold the partial rows)
+  int split;          // prefill_split_kernel: most key parts of an item (ws_o, ws_ml hold the partial rows)
+  int split_tiles;    //   and the fewest 64-key tiles of a sequence whose items are split
   const void* px_part;  // S normalised prefix parts [S][batch * n_q][D] of the head_dim type
   const float* px_lse;  // and their log2-domain log-sum-exp [S][batch * n_q]
   int px_n;             // S: the decode and its merge fold the parts into every row

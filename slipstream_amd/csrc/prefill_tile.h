@@ -116,9 +116,9 @@ __device__ __forceinline__ void wait_vm() {
 // twice, two parts of 12 tiles 25.1 against 27.8 us, over 600, 14 tiles, 28.0 both; 256 over 460 once,
 // four parts 24.2 against 23.0; 64 over 460 once, nine tiles in three parts 19.7 against 16.8).
 constexpr int kPartTiles = 3;
-__device__ __host__ __forceinline__ int split_least_tiles(int split) { return 8 + 12 / split; }
-__device__ __forceinline__ int split_part_tiles(int split, int tiles_all, int seq_tiles) {
-  return seq_tiles < split_least_tiles(split) ? max(tiles_all, 1) : max(kPartTiles, (seq_tiles + split - 1) / split);
+inline int split_least_tiles(int split) { return 8 + 12 / split; }  // p.split_tiles
+__device__ __forceinline__ int split_part_tiles(const AttnParams& p, int tiles_all, int seq_tiles) {
+  return seq_tiles < p.split_tiles ? max(tiles_all, 1) : max(kPartTiles, (seq_tiles + p.split - 1) / p.split);
 }
 
 extern __shared__ __attribute__((aligned(1024))) char s_tile_stages[];
@@ -190,7 +190,7 @@ __device__ __forceinline__ void prefill_tile_body(const AttnParams& p, const int
   const int kv_all = p.noncausal ? kvt : min(kvt, ctx - qlen + last_row / p.n_rep + 1);
   const int tiles_all = kv_all > 0 ? (kv_all + C::KT - 1) / C::KT : 0;
   // this workgroup's tiles [t0, ntiles): all of them, or its part
-  const int per_part = SPLIT ? split_part_tiles(p.split, tiles_all, (kvt + C::KT - 1) / C::KT) : tiles_all;
+  const int per_part = SPLIT ? split_part_tiles(p, tiles_all, (kvt + C::KT - 1) / C::KT) : tiles_all;
   const int t0 = SPLIT ? part * per_part : 0;
   if (SPLIT && part > 0 && t0 >= tiles_all) return;
   const bool partial = SPLIT && tiles_all > per_part;
