@@ -65,7 +65,11 @@ __device__ __forceinline__ u32x4 dequant_pairs(uint32_t w, uint32_t magic, float
 // compiler moved half of the accumulators between register files in every stage. What it
 // therefore does not look after: the operands come from LDS reads it does wait for and
 // from VALU results many instructions old, an accumulator is touched once per key step,
-// and mfma_drain stands between the last product and the first use of the results.
+// and between a stage's last product and anything that follows the loop (after it the
+// compiler copies accumulators wherever it likes) stand the barrier and the rotation of the
+// stages' registers: over twenty instructions, where eleven cycles are needed. (An s_nop of
+// that length in every stage took 2 % of the time.) tests/test_panel_code.py counts them in
+// the compiled code.
 template <typename T>
 __device__ __forceinline__ void mfma_acc(f32x4& acc, u32x4 a, u32x4 b) {
   if constexpr (sizeof(T) == 2 && __is_same(T, bf16_t))
@@ -73,8 +77,6 @@ __device__ __forceinline__ void mfma_acc(f32x4& acc, u32x4 a, u32x4 b) {
   else
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
-__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
-
 // Position of 16-byte chunk c of row r within the row's 128 LDS bytes: c ^ panel_swizzle(r).
 // A 16-byte LDS read runs in four passes of sixteen lanes, lanes 0-3, 12-15, 20-27 first,
 // then 4-11, 16-19, 28-31, and the same of the upper half: a pass takes rows 0-3 and 12-15
@@ -299,11 +301,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     sb1 = sb2;
     zb1 = zb2;
   }
-  mfma_drain();
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)  // no read of an accumulator above the drain
-#pragma unroll
-    for (int ns = 0; ns < NS; ++ns) asm volatile("" : "+a"(acc[mt][ns]));
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA into LDS is left when the workgroup ends
 
   // ---- results: lane holds C[m0 + 16 mt + ln][nb + 4 NS kg + 4 ns + e]
