@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64 * kMaxKW) void w4a16_kernel(const W4Params p) {
   // the table behind one memory round trip per entry).
   {
     const int esize = p.sdt == SS_DTYPE_F32 ? 4 : 2;
-    const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(p.sc, (uint32_t)((int64_t)p.n * p.groups * esize));
+    const __amdgpu_buffer_rsrc_t rsc = scale_rsrc(p, esize);
     const __amdgpu_buffer_rsrc_t rzp = buffer_rsrc(p.qz, (uint32_t)((int64_t)p.n * p.groups * 4));
     const int total = 16 * NS * p.groups;
     for (int q0 = threadIdx.x; q0 < total; q0 += 8 * blockDim.x) {
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(2, 2)))
   constexpr int TB = 8;
   const int esize = p.sdt == SS_DTYPE_F32 ? 4 : 2;
   const uint32_t f16_mask = p.sdt == SS_DTYPE_F16 ? ~0u : 0u, bf16_mask = p.sdt == SS_DTYPE_BF16 ? ~0u : 0u;
-  const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(p.sc, (uint32_t)((int64_t)p.n * p.groups * esize));
+  const __amdgpu_buffer_rsrc_t rsc = scale_rsrc(p, esize);
   const __amdgpu_buffer_rsrc_t rzp = buffer_rsrc(p.qz, (uint32_t)((int64_t)p.n * p.groups * 4));
   const int total = TR * gr;
   uint32_t sbits[TB];
@@ -1085,7 +1085,7 @@ __global__ __launch_bounds__(LB) void w4a16_skinny_kernel(const W4Params p) {
   // scales of esize bytes and ST int32 zero points, contiguous in each row
   const int esize = p.sdt == SS_DTYPE_F32 ? 4 : 2;
   const uint32_t f16_mask = p.sdt == SS_DTYPE_F16 ? ~0u : 0u, bf16_mask = p.sdt == SS_DTYPE_BF16 ? ~0u : 0u;
-  const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(p.sc, (uint32_t)((int64_t)p.n * p.groups * esize));
+  const __amdgpu_buffer_rsrc_t rsc = scale_rsrc(p, esize);
   const __amdgpu_buffer_rsrc_t rzp = buffer_rsrc(p.qz, (uint32_t)((int64_t)p.n * p.groups * 4));
   // ST fp32 scales, or ST 16-bit scales from the dword holding the first (ST / 2 + 1
   // dwords cover them whether that one starts at a low or a high half). The same NSD
@@ -1337,7 +1337,7 @@ __global__ __launch_bounds__(512) void w4a16_gemv_kernel(const W4Params p) {
     xin[e2] = r < p.m ? load16((const T*)p.x + (int64_t)r * p.x_stride + 8 * c8) : z;
   }
   const int esize = p.sdt == SS_DTYPE_F32 ? 4 : 2;
-  const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(p.sc, (uint32_t)((int64_t)p.n * p.groups * esize));
+  const __amdgpu_buffer_rsrc_t rsc = scale_rsrc(p, esize);
   const __amdgpu_buffer_rsrc_t rzp = buffer_rsrc(p.qz, (uint32_t)((int64_t)p.n * p.groups * 4));
   uint32_t sb[IT];
   int zi[IT];
@@ -1500,7 +1500,7 @@ __global__ __launch_bounds__(512) void w4a16_narrow_kernel(const W4Params p) {
   static_assert(IT == 8 || IT == 16, "two or four groups per lane in the scale block");
   static_assert(SD >= 0, "a fixed scale dtype");
   constexpr int esize = SD == SS_DTYPE_F32 ? 4 : 2;
-  const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(p.sc, (uint32_t)((int64_t)p.n * p.groups * esize));
+  const __amdgpu_buffer_rsrc_t rsc = scale_rsrc(p, esize);
   const __amdgpu_buffer_rsrc_t rzp = buffer_rsrc(p.qz, (uint32_t)((int64_t)p.n * p.groups * 4));
   constexpr int LPR = 16 / J;  // lanes per row
   const int lr = lane / LPR, lh = lane - lr * LPR;
@@ -2283,6 +2283,9 @@ extern "C" int ss_w4a16_gemm(const void* x, void* out, const int32_t* qweight, c
   if (pl.fast && ((int64_t)63 * x_stride + k) * 2 >= ((int64_t)1 << 31)) pl.fast = false;
   // scale and zero-point offsets are 32-bit byte offsets
   if (pl.fast && n * (k / group_size) * 4 >= ((int64_t)1 << 31)) pl.fast = false;
+  // 16-bit scales are read by the dword (scale_rsrc)
+  if (pl.fast && scale_dtype != SS_DTYPE_F32 && n * (k / group_size) % 2 != 0 && ((uintptr_t)scales & 3) != 0)
+    pl.fast = false;
   if (pl.fast && (pl.tile || pl.widek || pl.panel) && pl.ks > 1) {
     // the K split needs the workspace ss_w4a16_workspace_size reports; without it (or
     // unaligned) the wide kernel's plan if it does not split, else the untiled MFMA

@@ -103,9 +103,8 @@ __device__ __forceinline__ float load_scale(const void* s, int64_t i, int sdt) {
 
 // Scales read without branching on their dtype around the load (a load inside a
 // dtype branch makes the compiler wait for every outstanding load at the join):
-// the aligned dword holding scale gi, through a descriptor bounded by the array
-// (bytes past its end read as zero), shifted so the scale's bits are the low ones;
-// decoded afterwards.
+// the aligned dword holding scale gi, through a descriptor over the array (scale_rsrc),
+// shifted so the scale's bits are the low ones; decoded afterwards.
 __device__ __forceinline__ uint32_t scale_bits(__amdgpu_buffer_rsrc_t rs, int64_t gi, int esize) {
   const int off = (int)(gi * esize);
   return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, off & ~3, 0, 0) >> (8 * (off & 2));
@@ -180,6 +179,13 @@ __device__ __forceinline__ float dot2_acc<f16_t>(uint32_t a, uint32_t b, float a
 // address arithmetic.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
+}
+
+// Over the scales, their last dword counted whole: a dword that reaches past the descriptor
+// comes back as zero, and with it the last of an odd number of 16-bit scales. (The array is
+// then 4-byte aligned, host-checked, so that the dword lies in one page.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t scale_rsrc(const W4Params& p, int esize) {
+  return buffer_rsrc(p.sc, ((uint32_t)((int64_t)p.n * p.groups * esize) + 3u) & ~3u);
 }
 
 constexpr int kOutOfRange = 0x40000000;  // buffer offset past any operand (< 2^31 bytes)

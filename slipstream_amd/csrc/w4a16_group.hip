@@ -61,7 +61,7 @@ __global__ __launch_bounds__(1024) void w4a16_group_kernel(const W4Params p, int
 
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(p.qw, (uint32_t)((int64_t)p.n * p.k / 2));
   const int esize = p.sdt == SS_DTYPE_F32 ? 4 : 2;
-  const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(p.sc, (uint32_t)((int64_t)p.n * p.groups * esize));
+  const __amdgpu_buffer_rsrc_t rsc = scale_rsrc(p, esize);
   const __amdgpu_buffer_rsrc_t rzp = buffer_rsrc(p.qz, (uint32_t)((int64_t)p.n * p.groups * 4));
   const uint32_t f16_mask = p.sdt == SS_DTYPE_F16 ? ~0u : 0u, bf16_mask = p.sdt == SS_DTYPE_BF16 ? ~0u : 0u;
   const __amdgpu_buffer_rsrc_t rx = buffer_rsrc(

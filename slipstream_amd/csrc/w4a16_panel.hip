@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // ---- scale and zero point of the wave's rows at one stage, one row per lane, turned
   // around through the wave's own table
   const int esize = p.sdt == SS_DTYPE_F32 ? 4 : 2;
-  const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(p.sc, (uint32_t)((int64_t)p.n * p.groups * esize));
+  const __amdgpu_buffer_rsrc_t rsc = scale_rsrc(p, esize);
   const __amdgpu_buffer_rsrc_t rzp = buffer_rsrc(p.qz, (uint32_t)((int64_t)p.n * p.groups * 4));
   const int g_row = min(nb + lane % WR, p.n - 1) * p.groups;
   const uint32_t f16_mask = p.sdt == SS_DTYPE_F16 ? ~0u : 0u, bf16_mask = p.sdt == SS_DTYPE_BF16 ? ~0u : 0u;

@@ -280,6 +280,28 @@ def test_rows_past_64_keep_the_untiled_kernel(device, m, k, g):
     assert torch.equal(w4a16_gemm(xd, qd[:4096], sd[:4096], zd[:4096], g), y[:, :4096])
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("m,k,n,g,act,sdt", [
+    (3, 128, 357, 128, torch.bfloat16, torch.float16),    # skinny kernel, one group
+    (12, 640, 277, 128, torch.float16, torch.bfloat16),   # skinny, five
+    (1, 1152, 99, 128, torch.bfloat16, torch.bfloat16),   # group kernel
+    (20, 2432, 4467, 128, torch.float16, torch.float16),  # untiled
+    (187, 896, 393, 128, torch.bfloat16, torch.float16),
+    (94, 768, 575, 256, torch.float16, torch.bfloat16),   # tiled
+])
+def test_odd_number_of_scales(device, m, k, n, g, act, sdt, offset):
+    """An odd number of 16-bit scales: the last one, of the last weight row's last group, lies
+    in a dword that ends past the array. Also with the array 2 bytes off a dword."""
+    x, qw, s, z, ref = _host_case(n, k, m, g, seed=m + k + n, act=act, sdt=sdt, zeros="random")
+    assert s.numel() % 2 == 1
+    buf = torch.full((s.numel() + offset + 1,), float("nan"), device=device, dtype=sdt)
+    sd = buf[offset : offset + s.numel()].view(s.shape)
+    sd.copy_(s)
+    y = w4a16_gemm(x.to(device), qw.to(device), sd, z.to(device), g)
+    _assert_close(y, ref, f"odd scales m={m} k={k} n={n} g={g}")
+    _assert_close(y[:, -1:], ref[:, -1:], f"odd scales, the last column, m={m} k={k} n={n} g={g}")
+
+
 # (untiled forms as the host computes them for 256 CUs)
 @pytest.mark.parametrize("m,k,n,act,sdt,staged", [
     (1, 7296, 8240, torch.bfloat16, torch.float16, True),    # one row in LDS
