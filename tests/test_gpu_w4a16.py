@@ -405,8 +405,9 @@ def test_wide_kernel_two_ranges_graph_and_dirty_workspace(device):
 
 def test_workspace_growth_keeps_a_captured_graphs_buffer(device):
     """A call that needs a larger workspace than the stream's must not free the buffer a
-    graph captured earlier writes its partials to: the graph replays to its own result
-    after the growth, a cache trim and a fill of what was freed."""
+    graph captured earlier writes its partials to. After the growth, memory of that size
+    allocated on the stream and filled is not the old buffer: the graph replays to its own
+    result and leaves the fill alone."""
     from slipstream_amd.kernels import quant_gemm
     small = workloads.w4a16_linear(8192, 2048, 64, device=device, seed=1)   # split K, a few MB of partials
     large = workloads.w4a16_linear(8192, 6144, 256, device=device, seed=2)
@@ -416,26 +417,59 @@ def test_workspace_growth_keeps_a_captured_graphs_buffer(device):
     def call(lin):
         return w4a16_gemm(lin.x, lin.qweight, lin.scales, lin.qzeros, lin.group_size)
 
+    key = (torch.device(device).index or 0, st.cuda_stream)
+    quant_gemm._WORKSPACE.pop(key, None)  # another stream's, had it the same handle
     with torch.cuda.stream(st):
         want = call(small)
     st.synchronize()
-    key = (torch.device(device).index or 0, st.cuda_stream)
-    before = quant_gemm._WORKSPACE[key]
+    # the buffer's address and size alone: a reference to it here would keep it alive
+    ptr, size = quant_gemm._WORKSPACE[key].data_ptr(), quant_gemm._WORKSPACE[key].numel()
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, stream=st):
         out = call(small)
     with torch.cuda.stream(st):
         call(large)
     st.synchronize()
-    after = quant_gemm._WORKSPACE[key]
-    assert after.numel() >= 2 * before.numel() or after is before
-    assert after is before or any(r is before for r in quant_gemm._RETIRED)
+    grown = quant_gemm._WORKSPACE[key]
+    assert grown.data_ptr() != ptr and grown.numel() >= 2 * size
+    assert any(r.data_ptr() == ptr and r.numel() == size for r in quant_gemm._RETIRED)
+    with torch.cuda.stream(st):
+        fill = [torch.full((size,), 0xFF, dtype=torch.uint8, device=device) for _ in range(3)]
     for _ in range(3):
         out.zero_()
         torch.cuda.synchronize()
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+        assert all(bool((f == 0xFF).all()) for f in fill)
+
+
+@pytest.mark.parametrize("m,k,n,act", [
+    (150, 8192, 4100, torch.bfloat16),   # seven K ranges on the panel kernel
+    (70, 4096, 16388, torch.float16),    # three
+    (600, 4096, 3074, torch.bfloat16),   # two, N % 4 != 0
+])
+def test_panel_without_its_workspace(device, m, k, n, act):
+    """Where the panel kernel splits K, a call without the workspace, with one too small or off
+    16 bytes takes kernels that need less, to the same tolerance; with it, to the Python
+    call's bits."""
+    from slipstream_amd import _ffi
+    x, qw, s, z, ref = _host_case(n, k, m, 128, seed=m + k + n, act=act, zeros="random")
+    xd, qd, sd, zd = x.to(device), qw.to(device), s.to(device), z.to(device)
+    lib, code = _ffi.lib(), _ffi.dtype_code(act)
+    need = _ffi.ctypes.c_int64(0)
+    assert lib.ss_w4a16_workspace_size(m, n, k, 128, code, _ffi.ctypes.byref(need)) == _ffi.SS_OK
+    assert need.value >= 2 * m * n * 4
+    ws = torch.empty(need.value + 16, dtype=torch.uint8, device=device)
+    for ptr, size in ((ws.data_ptr(), need.value), (None, 0), (ws.data_ptr(), need.value // 2),
+                      (ws.data_ptr(), m * n * 4 - 1), (ws.data_ptr() + 8, need.value)):
+        y = torch.full((m, n), float("nan"), dtype=act, device=device)
+        st = lib.ss_w4a16_gemm(xd.data_ptr(), y.data_ptr(), qd.data_ptr(), sd.data_ptr(), zd.data_ptr(), m, n, k, 128,
+                               k, n, code, _ffi.dtype_code(sd.dtype), ptr, size, _ffi.stream_ptr(xd.device))
+        assert st == _ffi.SS_OK, lib.ss_last_error()
+        _assert_close(y, ref, f"panel m={m} k={k} n={n} workspace {size}")
+        if ptr == ws.data_ptr() and size == need.value:
+            assert torch.equal(y, w4a16_gemm(xd, qd, sd, zd, 128))
 
 
 def test_tiled_uneven_ranges_from_the_table_cap(device):
