@@ -12,7 +12,11 @@
 //
 // An MFMA of 16x16x32 must stay inside one quantisation group for the fp32 fold
 //     acc += s G - s (MAGIC + z) X,  G = sum x (MAGIC + q),  X = sum x,
-// but a lane's 16-byte weight load is 32 consecutive keys of its row. The four lanes of a
+// which groups of 64 keys take every 32 as smaller groups do: the MAGIC part that cancels
+// carries the rounding of G and X, and grows with their length (fp16, folded per 64: 6.3 %
+// of the results of 896 x 9728 not the nearest to the exact sum, per 32 5.5 %).
+//
+// A lane's 16-byte weight load is 32 consecutive keys of its row. The four lanes of a
 // row hold four such runs, and a 4 x 4 exchange of their words (two v_permlane32_swap, two
 // v_permlane16_swap) gives each lane the words of keys 32 s + 8 kg in step s.
 //
@@ -39,12 +43,13 @@ __device__ __forceinline__ u32x4 exchange_words(u32x4 w) {
   return u32x4{c[0], c[1], d[0], d[1]};
 }
 
-// GS: 32-key MFMA steps per fold unit, which lies in one quantisation group (4: g % 128 ==
-// 0, 2: g == 64, 1: any other g % 32 == 0); per: stages of a wave's run.
+// GS: 32-key MFMA steps per scale, all in one quantisation group (4: g % 128 == 0, 2: g ==
+// 64, 1: any other g % 32 == 0); per: stages of a wave's run.
 template <typename T, int MT, int NS, int GS, int P>
 __global__ __launch_bounds__(1024) void w4a16_group_kernel(const W4Params p, int per) {
   typedef W4Elem<T> E;
   constexpr int NG = 4 / GS;   // groups of a stage
+  constexpr int FS = GS == 4 ? 4 : 1;  // steps of a fold
   constexpr int NGR = P * NG;  // and of a round
   constexpr int EL = (NGR + 3) / 4;  // of those, a lane's
   extern __shared__ __attribute__((aligned(16))) char s_dyn[];
@@ -78,7 +83,7 @@ __global__ __launch_bounds__(1024) void w4a16_group_kernel(const W4Params p, int
   for (int mt = 0; mt < MT; ++mt)
     x_off[mt] = (int)((int64_t)min(16 * mt + ln, rows - 1) * p.x_stride * (int64_t)sizeof(T)) + 16 * kg;
 
-  // quantisation group of fold unit e (32 GS keys each)
+  // quantisation group of the e-th 32 GS keys
   auto group_at = [&](int e) { return GS == 2 ? e : (int)((uint32_t)(e * (32 * GS)) / (uint32_t)p.g); };
   const uint32_t magic = in_vgpr(E::kMagicPair);
   const u32x4 ones = {E::kOnePair, E::kOnePair, E::kOnePair, E::kOnePair};
@@ -138,7 +143,7 @@ __global__ __launch_bounds__(1024) void w4a16_group_kernel(const W4Params p, int
       f32x4 G[MT][NS], X[MT];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        if (s % GS == 0) {
+        if (s % FS == 0) {
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
             X[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -157,7 +162,7 @@ __global__ __launch_bounds__(1024) void w4a16_group_kernel(const W4Params p, int
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) G[mt][ns] = Elem<T>::mfma(x[u][s][mt], b, G[mt][ns]);
         }
-        if (s % GS == GS - 1) {
+        if (s % FS == FS - 1) {
 #pragma unroll
           for (int ns = 0; ns < NS; ++ns) {
             const float2 t = s_tab[(u * NG + s / GS) * 16 * NS + 16 * ns + ln];

@@ -280,6 +280,19 @@ def test_rows_past_64_keep_the_untiled_kernel(device, m, k, g):
     assert torch.equal(w4a16_gemm(xd, qd[:4096], sd[:4096], zd[:4096], g), y[:, :4096])
 
 
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,k,n", [(1, 896, 300), (11, 896, 9728), (16, 4864, 900), (30, 1152, 8200), (50, 896, 2000)])
+def test_group_kernel_folds_every_32_keys(device, m, k, n, act):
+    """Groups of 64 keys give the bits of the same weights in groups of 32 (each scale and zero
+    point twice): partial sums are folded every 32 keys, whose bias cancels with less rounding
+    than that of 64."""
+    x, qw, s, z, ref = _host_case(n, k, m, 64, seed=m + k, act=act, zeros="random")
+    xd, qd, sd, zd = x.to(device), qw.to(device), s.to(device), z.to(device)
+    y = w4a16_gemm(xd, qd, sd, zd, 64)
+    _assert_close(y, ref, f"g=64 m={m} k={k} n={n}")
+    assert torch.equal(y, w4a16_gemm(xd, qd, sd.repeat_interleave(2, 1), zd.repeat_interleave(2, 1), 32))
+
+
 @pytest.mark.parametrize("offset", [0, 1])
 @pytest.mark.parametrize("m,k,n,g,act,sdt", [
     (3, 128, 357, 128, torch.bfloat16, torch.float16),    # skinny kernel, one group
@@ -507,8 +520,9 @@ def test_tiled_without_workspace_takes_untiled_kernel(device):
     _assert_close(w4a16_gemm(xd, qd, sd, zd, g), ref, "with workspace")
 
 
-def test_large_scale_table_takes_scalar_kernel(device):
-    """k/group_size too large for the LDS scale table: the scalar kernel, same answer."""
+def test_large_scale_table_takes_group_kernel(device):
+    """k/group_size too large for the untiled kernel's LDS scale table: the group kernel, which
+    has none; same answer."""
     x, qw, s, z, ref = _host_case(32, 20480, 2, 32, seed=5, zeros="random")
     y = w4a16_gemm(x.to(device), qw.to(device), s.to(device), z.to(device), 32)
     _assert_close(y, ref, "k=20480 g=32")
