@@ -95,6 +95,11 @@ int ss_reshape_and_cache(const void* k, const void* v, void* k_cache, void* v_ca
  * 128-row query tile), so the size depends on batch and max_query_len then; the
  * general kernel's key-split partials (at most 2 x CUs x 16 x (head_dim + 2) x 4
  * bytes) fit inside the same size.
+ * A padded prefill of few (sequence, KV head, 128-row query tile) items splits the keys of
+ * long sequences over workgroups, and how often follows from the number of items, the block
+ * table's width and the workspace's size: a sequence's result is the same from call to call
+ * with those, but may differ in the last bits from the result in another batch, over a
+ * wider table or in the packed form (which never splits).
  */
 int ss_paged_attention_workspace_size(int64_t batch, int n_q, int n_kv, int head_dim,
                                       int max_query_len, int dtype, int64_t* bytes);

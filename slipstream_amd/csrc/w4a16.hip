@@ -1654,7 +1654,9 @@ bool plan_tile(W4Plan& pl, int64_t m, int64_t n, int64_t k, int g) {
   // m <= 16 is weight-bandwidth bound and the untiled kernel shares activations
   // well enough there; for K < 8192 it measured faster (no reduction launch) up to
   // N = 14336 (11.5 vs 12.8 us at 4096 x 6144), the tiled one from N = 28672 (26.9 vs
-  // 30.9 us at 4096 x 28672, the stacked gate/up projection)
+  // 30.9 us at 4096 x 28672, the stacked gate/up projection). (Of these shapes the skinny
+  // kernel takes those it splits and the group kernel short ones, each where it is faster
+  // than the untiled kernel; neither was measured against this one here.)
   if (m <= 16 && k < 8192 && n < 24576) return false;
   int mt, ns, pf;
   if (m <= 16)
@@ -1888,7 +1890,9 @@ W4Plan plan_w4a16(int64_t m, int64_t n, int64_t k, int g, bool act16, bool allow
   if (allow_tile && plan_wide(pl, m, n, k, g)) {
     // the panel kernel (weights rounded to the operand type in the same way) where its
     // taller tiles come out ahead. The wide kernel takes 2.15 us a stage and round of one
-    // workgroup per CU (m = 197 and 512 x 4096 x 28672: 2.2 us).
+    // workgroup per CU with two weight tiles a wave (m = 197 and 512 x 4096 x 28672: 2.2 us);
+    // with one it takes 1.5 us (197 x 14336 x 4096: 45 us for 28 stages), not the half priced
+    // here, so these shapes keep the wide kernel at times where the panel kernel would win.
     const int64_t xcd_cus = std::max(1, ss_host::device_cu_count() / 8);  // whole pairs go to one XCD
     const int64_t rounds = (((int64_t)pl.ks * pl.n_tiles + 7) / 8 * pl.m_blocks + xcd_cus - 1) / xcd_cus;
     double t = (double)rounds * (2.15 * pl.kchunk * pl.ns / kWideNS + 4.0);
@@ -1970,8 +1974,6 @@ unsigned long long next_arrival_tag() {
   return t;
 }
 
-// NS weight tiles per wave, WV waves: the plan's 64 * pl.ns rows per workgroup are
-// 16 * NS * WV
 // The K ranges' partials added in range order into the output.
 template <typename T>
 int launch_splitk_reduce(const W4Params& p, int ks, const float* part, hipStream_t stream) {
@@ -1987,6 +1989,8 @@ int launch_splitk_reduce(const W4Params& p, int ks, const float* part, hipStream
   return ss_host::launch_status("w4a16 split-K reduce");
 }
 
+// NS weight tiles per wave, WV waves: the plan's 64 * pl.ns rows per workgroup are
+// 16 * NS * WV
 template <typename T, int MT, int NS, int PF, int WV>
 int launch_w4a16_tile(const W4Params& p, const W4Plan& pl, float* part, hipStream_t stream) {
   if (16 * NS * WV != 64 * pl.ns) {

@@ -27,7 +27,7 @@
 // past the buffers; repeating a live stage instead cost 8.9 -> 9.8 us).
 //
 // Measured (m = 11, g = 64, weights from HBM) against the untiled kernel's activation
-// staging and scale tables: 896 x 9728 16.1 -> 5.7 us, 4864 x 896 25.8 -> 8.1 us. What is left
+// staging and scale tables: 896 x 9728 16.1 -> 5.8 us, 4864 x 896 25.8 -> 8.3 us. What is left
 // are the launch, one round trip to HBM and the LDS pass (0.3-0.9 TB/s of weights).
 #include "w4a16_common.h"
 

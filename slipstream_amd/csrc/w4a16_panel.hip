@@ -13,10 +13,12 @@
 //     eight waves reading, make its LDS reads as long as its MFMAs).
 // Activations come into LDS by DMA in half stages of 64 keys, a ring of four: one being
 // read, one landed (so that fragments are read ahead across the barrier), two on their
-// way. One wave per SIMD has nothing to hide behind, so the order is written out: every
-// MFMA is followed by an instruction or two of the next key step's dequantisation, at
-// times a fragment read six tiles ahead, a DMA instruction or a weight load (weights two
-// stages ahead), and the scheduler is held to that order.
+// way; at a stage's end, though, the compiler's waits for the scale and zero-point
+// loads, which it cannot tell from the DMAs behind them, leave none on its way. One
+// wave per SIMD has nothing to hide behind, so the order is written out: every MFMA is
+// followed by an instruction or two of the next key step's dequantisation, at times a
+// fragment read six tiles ahead, a DMA instruction or a weight load (weights two stages
+// ahead), and the scheduler is held to that order.
 //
 // The weights are the MFMA's row operand, so a lane's accumulators are consecutive output
 // columns; with tile row i of wave tile ns holding weight row 4 NS (i / 4) + 4 ns + i % 4 they
@@ -39,7 +41,8 @@ constexpr int kPanelTab = 4 * 2 * 64 * 8;  // LDS bytes of the four waves' scale
 // Eight int4 weights (one word: keys 8j .. 8j + 7 of a row) -> T((q - z) s) in key order.
 // A nibble OR-ed into the mantissa of fp16 1024 is 1024 + q, and an FMA reads either fp16
 // half in place: (1024 + q) s - (1024 + z) s. For 16-bit scales the constant is exact in
-// fp32, so the FMA gives (q - z) s, rounded once to T. Nineteen instructions a word (the
+// fp32 (zero points to 7167; finite for scales below 3e35), so the FMA gives (q - z) s,
+// rounded once to T. Nineteen instructions a word (the
 // byte converts of dequant_word take 23).
 template <int HALF>
 __device__ __forceinline__ void fma_half(uint32_t t, float s, float c, float& r) {

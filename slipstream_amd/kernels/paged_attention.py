@@ -283,6 +283,12 @@ def paged_attention_prefill(
     (``attention.py:44-45``); that check reads ``seq_lens`` on the host, so it is
     off by default and such rows then follow the Triton rule (rows with no
     visible key are zero).
+
+    A call of few sequences and tokens splits the keys of long sequences over workgroups,
+    by the number of (sequence, KV head, 128-row query tile) items and the width of
+    ``block_tables``: repeated calls give the same bits, but a sequence's result may differ
+    in the last bits from the same sequence in another batch, over a wider table or in
+    ``paged_attention_varlen``.
     """
     if _debug() and q.ndim == 4 and q.shape[2] > 1 and seq_lens.numel() > 0:
         shortest = int(seq_lens.min().item())
