@@ -1104,7 +1104,10 @@ __device__ __forceinline__ void decode_merge_body(const AttnParams& p, const int
     // round trip per batch), then merged into the running (max, sum, output). A sequence of
     // a small batch is cut into many pieces (23 of 179 keys for 4096 tokens of 37
     // sequences), so beyond four they go eight at a time (with a thread for every output,
-    // that call 42.2 -> 41.0 us; 256 sequences to 8192 tokens, few pieces each, 246.4 both).
+    // that call 42.2 -> 40.3 us; 256 sequences to 8192 tokens, few pieces each, 246.4 both).
+    // Nine to twelve are three rounds of four: in two of eight up to seven loads repeat the
+    // last piece (64 sequences behind a shared prefix of 736 tokens, 28/4 heads, 22.6 against
+    // 23.8 us).
     float mmax = kNegBig, lsum = 0.f;
     f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
     auto merge = [&](auto batch) __attribute__((always_inline)) {
@@ -1138,7 +1141,7 @@ __device__ __forceinline__ void decode_merge_body(const AttnParams& p, const int
         mmax = mx;
       }
     };
-    if (np <= 4)
+    if (np <= 4 || (np > 8 && np <= 12))
       merge(std::integral_constant<int, 4>{});
     else
       merge(std::integral_constant<int, 8>{});
